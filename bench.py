@@ -6,7 +6,9 @@
 
 A step is one call of mamba2_jax.kernels.mamba_chunk_scan_combined_fwd on
 synthetic inputs already resident in HBM, returning the output and the final
-states.  For bf16 at the benchmark shapes the five stages run as three kernels:
+states.  For bf16 at the headline shape the five stages run as two kernels:
+chunk_cumsum + bmm_chunk (side by side in one launch) and a walk over the
+chunks that does the rest; other bf16 shapes and packed sequences as three:
 chunk_cumsum (+ chunk-state weights), chunk_state + state_passing (one
 chunk-sequential kernel) and bmm_chunk + chunk_scan (one kernel).  Prints ONE
 JSON line (rank 0): tokens/s and ms per layer (W warm-up steps, then K
@@ -124,6 +126,37 @@ def stage_work(cfg, with_init=False, with_z=False, cu_seqlens=None):
     return w
 
 
+def walk_work(cfg, plan, with_init=False, with_z=False):
+    """stage_work of the one-pass layer (m2_ssd_combined_plan != 0): chunk_cumsum
+    and CB for chunks of 64 in one launch, then the walk; with several segments
+    per chain their end states (x and B read twice, the states written and
+    read) fall in the walk's interval."""
+    b, L, H, G, P, N = cfg.batch, cfg.seqlen, cfg.nheads, cfg.ngroups, cfg.headdim, cfg.dstate
+    nc, nseg = math.ceil(L / 64), plan // 2
+    cq, cb = b * H * nc * 64, b * nc * G * 10 * 512
+    xb, bb, st = 2 * b * L * H * P, 2 * b * L * G * N, 4 * b * H * P * N
+    prep = (2 * b * L * H + 12 * cq + 8 * H + 2 * bb + cb, 8 * b * L * H + 2 * b * nc * G * 10 * 256 * N)
+    by = (xb * (2 if with_z else 1) + 2 * bb + cb + 12 * cq + 4 * H + 2 * xb + st * (2 if with_init else 1)
+          + (xb + bb + 2 * st * (nseg - 1) if nseg > 1 else 0))
+    fl = b * nc * H * P * 64 * 65 + 4 * b * L * H * N * P * (1 if nseg == 1 else 1.5)
+    return {WALK_PREP: prep, WALK: (by, fl)}
+
+
+def layer_plan(cfg, kw):
+    """m2_ssd_combined_plan for a configuration's inputs."""
+    import ctypes
+    from mamba2_jax import _lib as L
+    set_ = lambda v: None if v is None else 16
+    a = L.SsdCombinedArgs(batch=cfg.batch, seqlen=cfg.seqlen, nheads=cfg.nheads, headdim=cfg.headdim,
+                          ngroups=cfg.ngroups, dstate=cfg.dstate, chunk_size=cfg.chunk_size,
+                          dtype=0 if cfg.dtype == "f32" else 1, dt_dtype=0 if cfg.dtype == "f32" else 1,
+                          dt_softplus=1, dt_min=0.0, dt_max=float("inf"), z=set_(kw.get("z")),
+                          seq_idx=set_(kw.get("seq_idx")), varlen_states=set_(kw.get("cu_seqlens")))
+    return L.load_library().m2_ssd_combined_plan(ctypes.byref(a))
+
+
+WALK_PREP = "chunk_cumsum+bmm_chunk"
+WALK = "layer_walk"
 FUSED_STATES = "chunk_state+state_passing"
 FUSED_CUMSUM = "chunk_cumsum+chunk_state"
 FUSED_PASS_BMM = "state_passing+bmm_chunk"
@@ -425,7 +458,7 @@ def bench_fp32_same_shape(cfg, name="c2", steps=100, warmup=50):
     c32 = dataclasses.replace(cfg, dtype="f32")
     kw = _layer_inputs(c32)
     nev = 300
-    finish = stage_table_enqueue(c32, kw, nev, stage_events(c32, nev))
+    finish = stage_table_enqueue(c32, kw, nev, stage_events(c32, nev, layer_plan(c32, kw)))
     ms, _ = time_layer(kw, steps, warmup)
     stages, dom, roof, _, tot_by = finish()
     attach_traffic(roof, measured_traffic(f"{name}_f32"), dom)
@@ -540,7 +573,7 @@ def stage_table_enqueue(cfg, kw, steps, events=None):
     the result of stage_events(cfg, steps), made beforehand (creating them
     takes host time during which the GPU would idle)."""
     from mamba2_jax.kernels import mamba_chunk_scan_combined_fwd
-    hev, evs, keep, fs, fc = events or stage_events(cfg, steps)
+    hev, evs, keep, fs, fc = events or stage_events(cfg, steps, layer_plan(cfg, kw))
     for _ in range(3):
         mamba_chunk_scan_combined_fwd(**kw, _stage_events=evs[0])
     for i in range(steps):
@@ -548,10 +581,14 @@ def stage_table_enqueue(cfg, kw, steps, events=None):
     return lambda: _stage_table_finish(cfg, kw, steps, hev, evs, keep, fs, fc)
 
 
-def stage_events(cfg, steps):
-    """The HIP events of a stage_table pass of `steps` calls (host side only)."""
+def stage_events(cfg, steps, plan=0):
+    """The HIP events of a stage_table pass of `steps` calls (host side only);
+    `plan`: layer_plan of the inputs."""
     import dataclasses
     hev = HipEvents()
+    if plan:
+        keep = [True, True, False, False, False, True, False]
+        return hev, [[hev.new() if k else None for k in keep] for _ in range(steps)], keep, False, False
     icfg = dataclasses.replace(cfg, chunk_size=internal_chunk(cfg))
     fs, fc = states_is_fused(icfg), scan_is_fused(icfg)
     fcs, fpb = cumsum_in_state(icfg), pass_bmm_fused(icfg)
@@ -580,21 +617,26 @@ def _stage_table_finish(cfg, kw, steps, hev, evs, keep, fs, fc):
     slot_ms = [slot(e) for e in range(1, 7 if keep[6] else 6)]
     last = rec[-1]
     total = float(np.mean([hev.elapsed_ms(evs[i][0], evs[i][last]) for i in range(steps)]))
+    plan = layer_plan(cfg, kw)
     cu = kw.get("cu_seqlens")
-    work = stage_work(cfg, with_init=kw["initial_states"] is not None,
+    work = walk_work(cfg, plan, kw["initial_states"] is not None) if plan else stage_work(cfg, with_init=kw["initial_states"] is not None,
                       cu_seqlens=None if cu is None or not keep[6] else cu.cpu().tolist())
     slots = dict(zip(STAGES, slot_ms))
-    if fs:
+    if plan:
+        first = {WALK_PREP: slots["chunk_cumsum"]}
+    elif fs:
         first = {"chunk_cumsum": slots["chunk_cumsum"], FUSED_STATES: slots["chunk_state"]}
     elif not keep[1]:
         first = {FUSED_CUMSUM: slots["chunk_state"], "state_passing": slots["state_passing"]}
     else:
         first = {k: slots[k] for k in STAGES[:3]}
-    if fc:
+    if plan:
+        second = {WALK: slots["chunk_scan"]}
+    elif fc:
         second = {"bmm_chunk+chunk_scan": slots["chunk_scan"]}
     else:
         second = {k: slots[k] for k in STAGES[3:]}
-    if not fs and not keep[3]:
+    if not plan and not fs and not keep[3]:
         # state_passing and bmm_chunk in one launch (its time: the bmm interval)
         first.pop("state_passing")
         first[FUSED_PASS_BMM] = second.pop("bmm_chunk")
@@ -637,7 +679,7 @@ def bench_other_config(name, steps=200, warmup=20, cpu=True):
     # c0's, ~35 us, needs ~1100 steps)
     est, _ = time_layer(kw, 20, 5)
     nev = max(steps, 300, int(40.0 / max(est, 1e-3)))
-    finish = stage_table_enqueue(cfg, kw, nev, stage_events(cfg, nev))
+    finish = stage_table_enqueue(cfg, kw, nev, stage_events(cfg, nev, layer_plan(cfg, kw)))
     ms, _ = time_layer(kw, steps, warmup)
     stages, dom, roof, _, tot_by = finish()
     attach_traffic(roof, measured_traffic(name), dom)
@@ -715,7 +757,7 @@ def main(argv=None):
     kw = _layer_inputs(cfg)
     K = args.steps
     nev = max(K, args.event_steps)
-    events = stage_events(cfg, nev)
+    events = stage_events(cfg, nev, layer_plan(cfg, kw))
     res_extra = {}
     # The other measurements run first and the headline follows them with no
     # idle gap: besides their own figures they keep the GPU at its steady

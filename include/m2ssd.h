@@ -217,6 +217,12 @@ typedef struct {
                                        is recorded before events 4 and 5    */
 } m2_ssd_combined_args;
 size_t m2_ssd_combined_workspace_size(const m2_ssd_combined_args* a);
+
+/* The kernels m2_ssd_combined runs for these sizes, types and flags (pointers are
+ * only tested for NULL): 0 the staged or two-pass path; else the one-pass walk,
+ * 2 s + p - 1 for s segments of a chain and p workgroups per head.  For
+ * measurements. */
+int m2_ssd_combined_plan(const m2_ssd_combined_args* a);
 int m2_ssd_combined(const m2_ssd_combined_args* a, void* stream);
 
 /* ---------------------------------------------------------------------------
@@ -442,6 +448,10 @@ int m2_skinny_gemm_norm(const m2_skinny_gemm_norm_args* a, void* stream);
                                      1 one workgroup per (chunk, head); v >= 2
                                      one per (chunk, group, slice of v - 1 of
                                      the group's heads)                        */
+#define M2_KNOB_LAYER         4   /* bf16 layer: 1 the one-pass walk, a workgroup
+                                     per head, 2 per half head, 3 the state
+                                     pass and the scan; 2 s, 2 s + 1 (s >= 2)
+                                     the walk, whole / half heads, in s segments */
 int m2_set_dispatch_override(int knob, int value);
 
 /* thread-local message for the last non-zero return code of this thread */

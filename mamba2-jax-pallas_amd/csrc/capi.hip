@@ -26,7 +26,7 @@ int check_launch(const char* what) {
     return M2_OK;
 }
 
-constexpr int NKNOBS = 4;
+constexpr int NKNOBS = 5;
 static std::atomic<int> g_knob[NKNOBS];
 
 int dispatch_override(int knob) {
@@ -54,7 +54,7 @@ extern "C" const char* m2_last_error(void) { return m2::g_err; }
 extern "C" int m2_abi_version(void) { return M2SSD_ABI_VERSION; }
 
 extern "C" int m2_set_dispatch_override(int knob, int value) {
-    static const int maxval[m2::NKNOBS] = {3, 2, 1, 65};
+    static const int maxval[m2::NKNOBS] = {3, 2, 1, 65, 65};
     if (knob < 0 || knob >= m2::NKNOBS || value < 0 || value > maxval[knob])
         return m2::set_error(M2_ERR_INVALID, "m2_set_dispatch_override: knob %d value %d", knob,
                              value);
@@ -173,6 +173,11 @@ extern "C" size_t m2_ssd_combined_workspace_size(const m2_ssd_combined_args* a) 
     return layout_of(internal_args(*a)).total;
 }
 
+extern "C" int m2_ssd_combined_plan(const m2_ssd_combined_args* a) {
+    return !a || a->chunk_size <= 0 || a->batch <= 0 || a->seqlen <= 0 || !m2_dtype_size(a->dtype)
+               ? 0 : m2::ssd_walk_plan(internal_args(*a));
+}
+
 extern "C" int m2_ssd_combined(const m2_ssd_combined_args* ap, void* stream_) {
     if (!ap) return m2::set_error(M2_ERR_INVALID, "m2_ssd_combined: NULL args");
     return m2::ssd_combined_on(*ap, ap->workspace, ap->workspace_bytes, (hipStream_t)stream_);
@@ -207,6 +212,16 @@ int m2::ssd_combined_on(const m2_ssd_combined_args& a0, void* workspace, size_t 
     const bool scan_cb = layer_scan_builds_cb(a);   // fp32: CB built in the group scan
     if ((rc = record(a.stage_events, 0, s))) return rc;
 
+    if (m2::ssd_walk_plan(a)) {
+        // cumsum (+ weights) and CB in one launch, then the rest of the layer in
+        // one kernel: their times land in the first and the last event interval
+        float* wts = (float*)(ws + l.wts);
+        if ((rc = m2::launch_ssd_walk_prep(a, dA, dto, wts, passed, s))) return rc;
+        for (int i = 1; i < 5; ++i)
+            if ((rc = record(a.stage_events, i, s))) return rc;
+        if ((rc = m2::launch_ssd_walk(a, dA, dto, wts, passed, s))) return rc;
+        return record(a.stage_events, 5, s);
+    }
     if (m2::states_fused_supported(a)) {
         // cumsum (+ weights and decay), then chunk states and state passing in
         // one kernel: its time lands in the second event interval, the third is

@@ -94,6 +94,18 @@ int launch_scan_fused(const m2_ssd_combined_args& a, const float* dA, const floa
 // struct's own workspace fields are not read)
 int ssd_combined_on(const m2_ssd_combined_args& a, void* ws, size_t ws_bytes, hipStream_t stream);
 
+// the whole combined forward in one chunk-sequential pass (csrc/ssd_walk.hip):
+// bf16, head dim 64, dstate 64 / 128 / 256, no seq_idx; its chunks are of 64
+// positions whatever chunk_size is.  launch_ssd_walk_prep computes chunk_cumsum's
+// dA / dt / weights for those and CB (in the workspace slot of the passed states,
+// which also holds the segment states of launch_ssd_walk behind it).
+// ssd_walk_plan: 0 where the other kernels run, else 2 segments + row parts - 1.
+int ssd_walk_plan(const m2_ssd_combined_args& a);
+int launch_ssd_walk_prep(const m2_ssd_combined_args& a, float* dA, float* dt, float* wts, void* cb,
+                         hipStream_t stream);
+int launch_ssd_walk(const m2_ssd_combined_args& a, const float* dA, const float* dt,
+                    const float* wts, void* cb, hipStream_t stream);
+
 // chunk_state + state_passing of the combined forward in one chunk-sequential
 // pass, from the weights / decay of launch_chunk_cumsum_ex; writes the states
 // entering each chunk (in the input dtype) and the final states.  bf16 inputs
@@ -102,6 +114,7 @@ int ssd_combined_on(const m2_ssd_combined_args& a, void* ws, size_t ws_bytes, hi
 bool states_fused_supported(const m2_ssd_combined_args& a);
 int launch_states_fused(const m2_ssd_combined_args& a, const float* wts, const float* scl,
                         void* states_passed, hipStream_t stream);
+double states_cost(const m2_ssd_combined_args& a);
 bool states_fused_f32_supported(const m2_ssd_combined_args& a);
 int launch_states_fused_f32(const m2_ssd_combined_args& a, const float* wts, const float* scl,
                             void* states_passed, hipStream_t stream);

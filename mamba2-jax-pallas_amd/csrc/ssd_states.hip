@@ -624,6 +624,20 @@ StatesSplit states_split(const m2_ssd_combined_args& a) {
     return SPLIT_HALVES;
 }
 
+// The pass's time in us (bf16), to weigh it against the one-pass layer: per
+// chunk and round of workgroups, growing with the workgroups side by side
+// (measured inside the layer, halves: 0.8-1.0 us at 128, 1.2-1.6 at 256; pairs x
+// 128 columns 1.0 / 1.9 / 3.0-3.7 at 64 / 128 / 256).
+double states_cost(const m2_ssd_combined_args& a) {
+    const StatesSplit sp = states_split(a);
+    const double nc = (double)((a.seqlen + a.chunk_size - 1) / a.chunk_size) * (double)a.chunk_size / 128.0;
+    const int64_t wg = a.batch * a.nheads / (sp == SPLIT_HALVES ? 1 : 2) * (a.dstate / (sp == SPLIT_PAIR128 ? 128 : 64));
+    const int64_t cus = cu_count(), r = (wg + cus - 1) / cus;
+    const double f = (double)(r > 1 ? cus : wg) / (double)cus;
+    const double st = sp == SPLIT_HALVES ? 0.45 + 1.1 * f : sp == SPLIT_PAIR64 ? 0.4 + 2.4 * f : 0.4 + 3.8 * f;
+    return r * (3.0 + nc * st);
+}
+
 int launch_states_fused(const m2_ssd_combined_args& a, const float* wts, const float* scl,
                         void* passed, hipStream_t s) {
     if (a.dtype == M2_F32) return launch_states_fused_f32(a, wts, scl, passed, s);

@@ -160,7 +160,7 @@ ENTRY_POINTS = {
     "m2_skinny_gemm": SkinnyGemmArgs,
     "m2_skinny_gemm_norm": SkinnyGemmNormArgs,
 }
-OTHER_SYMBOLS = ("m2_ssd_combined_workspace_size", "m2_last_error", "m2_abi_version",
+OTHER_SYMBOLS = ("m2_ssd_combined_workspace_size", "m2_ssd_combined_plan", "m2_last_error", "m2_abi_version",
                  "m2_set_dispatch_override", "m2_ssd_combined_noalloc_prepare")
 
 # testing hook m2_set_dispatch_override: knob name -> (M2_KNOB_*, {choice: value})
@@ -169,6 +169,9 @@ KNOBS = {
     "f32_states": (1, {"fused": 1, "staged": 2}),
     "oneshot_heads": (2, {"1": 1}),
     "f32_scan": (3, {"per_head": 1, **{f"group{n}": n + 1 for n in range(1, 65)}}),
+    "layer": (4, {"walk": 1, "walk_half": 2, "two_pass": 3,
+                  **{f"walk_x{n}": 2 * n for n in range(2, 33)},
+                  **{f"walk_half_x{n}": 2 * n + 1 for n in range(2, 33)}}),
 }
 
 
@@ -206,6 +209,8 @@ def load_library(path=LIB_PATH):
             fn.restype = ctypes.c_int
         lib.m2_ssd_combined_workspace_size.argtypes = [ctypes.POINTER(SsdCombinedArgs)]
         lib.m2_ssd_combined_workspace_size.restype = ctypes.c_size_t
+        lib.m2_ssd_combined_plan.argtypes = [ctypes.POINTER(SsdCombinedArgs)]
+        lib.m2_ssd_combined_plan.restype = ctypes.c_int
         lib.m2_last_error.argtypes = []
         lib.m2_last_error.restype = ctypes.c_char_p
         lib.m2_abi_version.argtypes = []

@@ -1,0 +1,123 @@
+"""The one-pass layer (csrc/ssd_walk.hip) against the oracle where it can go
+wrong: one position to a few chunks of 64 with every remainder, each dstate, a
+whole head or half of one per workgroup, chains cut into segments (fewer chunks
+than asked for, a last segment that is shorter), initial states, the z gate, D
+per head dim, rising dA_cumsum; and the plan the library picks by itself.
+
+Tolerance: the bf16 bar of the layer, 2e-2 of the RMS (it holds CB and the
+states entering each chunk in bf16, as the other paths do)."""
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import TOL, announce, check, dev, tdtype
+from mamba2_jax import _lib as L
+from mamba2_jax import configs
+from mamba2_jax.kernels import mamba_chunk_scan_combined_fwd
+from oracle import ssd_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+PLANS = ["walk", "walk_half", "walk_x2", "walk_half_x3", "walk_x32"]
+# (batch, L, H, G, dstate, chunk, init, z, D per head dim)
+SHAPES = [
+    (1, 1, 2, 1, 128, 128, False, False, False),
+    (2, 63, 4, 2, 64, 64, True, False, True),
+    (1, 64, 4, 1, 256, 128, True, True, False),
+    (1, 65, 2, 1, 128, 256, False, True, True),
+    (3, 130, 6, 2, 128, 128, True, False, False),
+    (1, 447, 4, 1, 256, 64, False, False, True),
+    (1, 1000, 5, 1, 64, 128, True, True, True),
+    (2, 1088, 4, 4, 128, 256, True, False, False),
+]
+
+
+def _inputs(b, Lq, H, G, N, Q, init, z, dhp, seed):
+    cfg = configs.SSDConfig("walk", b, Lq, H, G, 64, N, Q, "bf16", init_state=init, seed=seed)
+    d = configs.make_ssd_inputs(cfg, with_z=z)
+    if dhp:
+        d["D"] = np.random.default_rng(seed).uniform(0.5, 1.5, (H, 64)).astype(np.float32)
+    d.pop("seq_idx"), d.pop("cu_seqlens")
+    T = tdtype("bf16")
+    t = {k: dev(v, T if k in ("x", "dt", "B", "C", "z") else None) for k, v in d.items()}
+    return d, t
+
+
+def _check_all(t, d, plans, decay_clamp=False, **kw):
+    want = O.ssd_combined(io_dtype="bf16", decay_clamp=decay_clamp, **d, **kw)
+    for plan in plans:
+        announce("walk", plan)
+        if plan is None:
+            got = mamba_chunk_scan_combined_fwd(**t, **kw)
+        else:
+            with L.dispatch_override("layer", plan):
+                got = mamba_chunk_scan_combined_fwd(**t, **kw)
+        check(got[0], want[0], TOL["bf16"], "out")
+        check(got[1], want[1], TOL["bf16"], "final_states")
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "-".join(str(int(v)) for v in s))
+def test_walk_matches_oracle(shape):
+    announce("walk shape", shape)
+    d, t = _inputs(*shape, seed=sum(shape[:5]))
+    _check_all(t, d, PLANS + [None], chunk_size=shape[5], dt_softplus=True, return_final_states=True)
+
+
+def test_walk_rising_dA():
+    """A > 0: dA_cumsum rises, and the chunk states' decay is clamped at 0 chunk by
+    chunk, so the oracle runs the walk's chunks of 64.  The oracle rounds C h_c to
+    bf16 before the factor exp(dA): with A <= 16 / 2000 and dt' < 2 a chunk's dA
+    stays below 64 * 2 * 8e-3 = 1, so that rounding grows to at most 2^-9 e = 5.4e-3
+    of the term (A 20 times larger, exp(dA) to e^20, put it at 4.9e-2)."""
+    d, t = _inputs(1, 300, 4, 2, 128, 64, False, False, False, seed=5)
+    d["A"] = np.abs(d["A"] / 2000).astype(np.float32)
+    t["A"] = dev(d["A"])
+    _check_all(t, d, ["walk", "walk_half_x3"], decay_clamp=True, chunk_size=64, dt_softplus=True,
+               return_final_states=True)
+
+
+def test_signed_dt_keeps_the_two_passes():
+    """dt' of both signs (no softplus, dt_limit below 0): the clamped decay depends
+    on the chunk size, so a forced walk is ignored and chunks of 128 stay 128."""
+    d, t = _inputs(1, 512, 8, 2, 128, 128, False, False, False, seed=5)
+    t["dt"] = 0.05 * t["dt"]
+    t["dt_bias"] = None
+    kw = dict(chunk_size=128, dt_limit=(-1.0, float("inf")), return_final_states=True)
+    outs = []
+    for plan in ("two_pass", "walk"):
+        with L.dispatch_override("layer", plan):
+            outs.append(mamba_chunk_scan_combined_fwd(**t, **kw))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
+def test_walk_large_decay():
+    """|dA| past 500 within a chunk: the decay factors underflow, none overflows."""
+    d, t = _inputs(1, 300, 4, 1, 128, 128, True, False, False, seed=6)
+    d["A"] = (d["A"] * 40).astype(np.float32)
+    t["A"] = dev(d["A"])
+    _check_all(t, d, ["walk", "walk_half_x3"], chunk_size=128, dt_softplus=True,
+               return_final_states=True)
+
+
+@pytest.mark.parametrize("dt32", [False, True])
+def test_walk_repeats_bit_identically(dt32):
+    """The same call twice, another shape between: identical outputs (the
+    workspace holds the other call's data); dt in bf16 and float32."""
+    _, t = _inputs(1, 4096, 48, 1, 128, 256, False, False, False, seed=7)
+    _, o = _inputs(2, 777, 16, 2, 256, 128, True, False, False, seed=8)
+    if dt32:
+        t["dt"] = t["dt"].float()
+    kw = dict(dt_softplus=True, return_final_states=True)
+    a = [v.clone() for v in mamba_chunk_scan_combined_fwd(chunk_size=256, **t, **kw)]
+    mamba_chunk_scan_combined_fwd(chunk_size=128, **o, **kw)
+    b = mamba_chunk_scan_combined_fwd(chunk_size=256, **t, **kw)
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
+def test_two_pass_still_matches():
+    """The state pass and the scan, which packed sequences take, at a shape the
+    walk would take."""
+    shape = (1, 1000, 8, 2, 128, 128, True, False, False)
+    d, t = _inputs(*shape, seed=9)
+    _check_all(t, d, ["two_pass"], chunk_size=128, dt_softplus=True, return_final_states=True)
