@@ -4,7 +4,8 @@
 // A decode step reads every projection weight once per token, so these
 // products are HBM-bound on the weights (M * K * N MACs for 2 * K * N bytes).
 // The weights are K-contiguous ([N, K], the layout torch.nn.functional.linear
-// takes), so each lane loads 8 consecutive k of one output column as one
+// takes).  Up to 16 rows run k_skinny_stream (below); k_skinny_gemm takes the
+// rest: each lane loads 8 consecutive k of one output column as one
 // 16-byte access, which is exactly a 16x16x32 bf16 MFMA's B-operand fragment.
 // One workgroup per 16 output columns (fewer where that leaves CUs idle); its
 // 4, 8 or 16 wavefronts (enough for ~2048 over the chip) split K and meet in
@@ -36,6 +37,23 @@ struct GemmArgs {
     int bias_bf16, y_bf16;
     int cw;                 // output columns per workgroup (<= 16)
 };
+
+// rows 16 t + 4 (lane >> 4) + i of column n (+ bias): D layout of a 16x16 MFMA
+M2_DEV void store_tile(const GemmArgs& a, const f32x4& v, int n, int t) {
+    float bv = 0.f;
+    if (a.bias)
+        bv = a.bias_bf16 ? (float)reinterpret_cast<const bf16*>(a.bias)[n]
+                         : reinterpret_cast<const float*>(a.bias)[n];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int m = 16 * t + 4 * ((threadIdx.x & 63) >> 4) + i;
+        if (m < a.M) {
+            const float r = v[i] + bv;
+            if (a.y_bf16) reinterpret_cast<bf16*>(a.y)[(int64_t)m * a.ldy + n] = (bf16)r;
+            else reinterpret_cast<float*>(a.y)[(int64_t)m * a.ldy + n] = r;
+        }
+    }
+}
 
 // MT 16-row tiles of x, NW wavefronts splitting K
 template <int MT, int NW>
@@ -103,24 +121,107 @@ __global__ void __launch_bounds__(NW * 64) k_skinny_gemm(GemmArgs a) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) acc[t][i] += o[i];
         }
-    // D layout: lane holds column n0 + (lane & 15), rows 16 t + 4 (lane >> 4) + i
     const int n = n0 + col;
     if (!colok || n >= a.N) return;
-    float bv = 0.f;
-    if (a.bias)
-        bv = a.bias_bf16 ? (float)reinterpret_cast<const bf16*>(a.bias)[n]
-                         : reinterpret_cast<const float*>(a.bias)[n];
 #pragma unroll
-    for (int t = 0; t < MT; ++t)
+    for (int t = 0; t < MT; ++t) store_tile(a, acc[t], n, t);
+}
+
+// ---------------------------------------------------------------------------
+// k_skinny_stream: the same product at up to 16 rows, for a weight stream as
+// deep as LDS allows.  A workgroup takes cw columns (CT tiles of 16) and splits K
+// over its NW wavefronts; each wavefront keeps the x fragments of its K range in
+// registers (2 PU k steps; every column tile reuses them) and streams its part
+// of the weights through a ring of D 2 KB units of its own by direct global ->
+// LDS loads: 16 columns (or, first, the rows of x) x 64 k, whole 128-byte lines.
+// No wavefront waits for
+// another before the final sum, and no load result passes through registers, so
+// up to D NW 2 KB = 128 KB per CU stay in flight; k_skinny_gemm holds 8 KB per
+// wavefront in 64-byte pieces and reads x again for every 16 columns.  Measured
+// alone at 16 rows, weights past the cache: 2560 x 10576 22.6 -> 12.2 us (4.4
+// TB/s), 5120 x 2560 12.7 -> 8.5, 2560 x 50288 83 -> 53 (4.9 TB/s), 1536 x 6448
+// 10.1 -> 6.5, 768 x 3352 4.45 -> 4.1 (of which ~3.5 any kernel takes).
+// ---------------------------------------------------------------------------
+template <int N> M2_DEV void wait_units(int later) {   // at most `later` <= N units in flight
+    if constexpr (N == 0) wait_vmem<0>();
+    else if (later >= N) wait_vmem<2 * N>();
+    else wait_units<N - 1>(later);
+}
+
+template <int CT, int PU, int NW, int D>
+__global__ void __launch_bounds__(NW * 64) k_skinny_stream(GemmArgs a) {
+    constexpr int NU = (1 + CT) * PU;                  // units of a wavefront: x, then the weights
+    __shared__ __align__(16) char ring[NW][D * 2048];
+    static_assert(CT * 1024 <= D * 2048, "the partial sums reuse the ring");
+    const int lane = threadIdx.x & 63, w = wave_id();
+    const int n0 = blockIdx.x * a.cw;
+    const int nc = min(a.cw, a.N - n0);                // this workgroup's columns
+    const int k0 = w * PU * 64;                        // this wavefront's K range
+    const int col = lane & 15, kg = lane >> 4;
+    // lane l of load i of a unit brings 16-byte chunk l % 8 (swizzled by the row)
+    // of the tile's row 8 i + l / 8; rows past the last column (the last row of x)
+    // repeat it, so that every unit is two loads
+    const int row = lane >> 3, ch = (lane & 7) ^ row;
+    uint32_t vo[1 + CT][2];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int m = 16 * t + 4 * (lane >> 4) + i;
-            if (m < a.M) {
-                const float v = acc[t][i] + bv;
-                if (a.y_bf16) reinterpret_cast<bf16*>(a.y)[(int64_t)m * a.ldy + n] = (bf16)v;
-                else reinterpret_cast<float*>(a.y)[(int64_t)m * a.ldy + n] = v;
-            }
+    for (int i = 0; i < 2; ++i) {
+        vo[0][i] = 2 * (uint32_t)(min(8 * i + row, a.M - 1) * a.ldx);
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+            vo[1 + c][i] = 2 * (uint32_t)(min(16 * c + 8 * i + row, nc - 1) * a.ldw);
+    }
+    const uint32_t ring_lds = lds_addr(&ring[w][0]);
+    const bf16* w0 = a.w + (int64_t)n0 * a.ldw;
+    auto issue = [&](int q) {                          // unit q: x or column tile q / PU - 1, 64 k from k
+        const int c = q / PU, k = k0 + 64 * (q % PU);
+        const bf16* base = c == 0 ? a.x : w0;
+        const uint32_t dst = ring_lds + (q % D) * 2048;
+        // (chunks past the end of K repeat the last one; masked below)
+        const bool whole = k + 64 <= a.K;
+        const bf16* src = whole ? base + k : base;
+        const uint32_t o = whole ? 16 * ch : 2 * min(k + 8 * ch, a.K - 8);
+        dma16s(src, vo[c][0] + o, dst);
+        dma16s(src, vo[c][1] + o, dst + 1024);
+    };
+#pragma unroll
+    for (int q = 0; q < (D < NU ? D : NU); ++q) issue(q);
+    f32x4 acc[CT];
+#pragma unroll
+    for (int c = 0; c < CT; ++c) acc[c] = zero4();
+    const int fo = (col & 7) * 128 + (col >> 3) * 1024;
+    const bf16x8 zf = {};
+    bf16x8 xf[2 * PU];
+#pragma unroll
+    for (int q = 0; q < NU; ++q) {
+        wait_units<D - 1>(NU - 1 - q);
+        const char* u = &ring[w][(q % D) * 2048] + fo;
+        bf16x8 bf[2];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+            bf[ks] = *reinterpret_cast<const bf16x8*>(u + (((4 * ks + kg) ^ (col & 7)) * 16));
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (q + D < NU) issue(q + D);                  // the slot just read
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            const int s = 2 * (q % PU) + ks;
+            if (k0 + 32 * s + 8 * kg >= a.K) bf[ks] = zf;        // past the end of K
+            if (q < PU) xf[s] = bf[ks];
+            else acc[q / PU - 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[s], bf[ks], acc[q / PU - 1], 0, 0, 0);
         }
+    }
+    // the K-split partial sums of tile c meet in wavefront c
+#pragma unroll
+    for (int c = 0; c < CT; ++c) *reinterpret_cast<f32x4*>(&ring[w][c * 1024 + 16 * lane]) = acc[c];
+    __syncthreads();
+    if (w >= CT) return;
+    f32x4 v = *reinterpret_cast<const f32x4*>(&ring[0][w * 1024 + 16 * lane]);
+#pragma unroll
+    for (int j = 1; j < NW; ++j) {
+        const f32x4 o = *reinterpret_cast<const f32x4*>(&ring[j][w * 1024 + 16 * lane]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] += o[i];
+    }
+    if (16 * w + col < nc) store_tile(a, v, n0 + 16 * w + col, 0);
 }
 
 constexpr int NORM_MAXM = 16;       // rows of the normalising GEMM (one row tile)
@@ -303,6 +404,45 @@ void launch_mt(const GemmArgs& k, int64_t ngroups, hipStream_t s) {
     }
 }
 
+// k_skinny_stream for up to 16 rows and K up to 8192 (8 units of x fragments in
+// each of 16 wavefronts): false where it does not apply.  8 wavefronts with
+// twice the ring each where several column tiles follow each other and a K range
+// is at most 6 units; 16 for a single tile, whose loads all go out at once.
+template <int CT, int NW, int D>
+bool launch_stream_pu(const GemmArgs& k, int pu, const dim3& grid, hipStream_t s) {
+#define M2_STREAM_PU(V)                                                                    \
+    case V:                                                                                \
+        hipLaunchKernelGGL((k_skinny_stream<CT, V, NW, D>), grid, dim3(NW * 64), 0, s, k); \
+        return true;
+    switch (pu) {
+        M2_STREAM_PU(1) M2_STREAM_PU(2) M2_STREAM_PU(3) M2_STREAM_PU(4) M2_STREAM_PU(5) M2_STREAM_PU(6)
+        M2_STREAM_PU(7) M2_STREAM_PU(8)
+        default: return false;
+    }
+#undef M2_STREAM_PU
+}
+
+bool launch_stream(GemmArgs k, hipStream_t s) {
+    const int64_t cus = m2::cu_count();
+    if (k.M > 16 || k.K > 8192 || k.ldx >= (1 << 24) || k.ldw >= (1 << 24)) return false;   // 32-bit offsets
+    // columns per workgroup: as even over whole rounds of the CUs as up to three
+    // tiles allow, at least 4
+    const int64_t r = (k.N + 48 * cus - 1) / (48 * cus);
+    const int64_t cw = (k.N + r * cus - 1) / (r * cus);
+    k.cw = (int)(cw < 4 ? 4 : cw);
+    const dim3 grid((unsigned)((k.N + k.cw - 1) / k.cw));
+    const int ct = (k.cw + 15) / 16, units = (k.K + 63) / 64;
+    const int nw = units > 8 * 6 || ct == 1 ? 16 : 8;
+    const int pu = (units + nw - 1) / nw;
+    if (nw == 16) {
+        if (ct == 1) return launch_stream_pu<1, 16, 4>(k, pu, grid, s);
+        if (ct == 2) return launch_stream_pu<2, 16, 4>(k, pu, grid, s);
+        return launch_stream_pu<3, 16, 4>(k, pu, grid, s);
+    }
+    if (ct == 2) return launch_stream_pu<2, 8, 8>(k, pu, grid, s);
+    return launch_stream_pu<3, 8, 8>(k, pu, grid, s);
+}
+
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 // Output columns per workgroup: 16 (a full MFMA tile) when that gives at
@@ -346,6 +486,7 @@ int launch_skinny_gemm(const m2_skinny_gemm_args& a, hipStream_t s) {
     k.ldx = a.ldx; k.ldw = a.ldw; k.ldy = a.ldy;
     k.M = (int)a.M; k.N = (int)a.N; k.K = (int)a.K;
     k.bias_bf16 = a.bias_dtype == M2_BF16; k.y_bf16 = a.y_dtype == M2_BF16;
+    if (launch_stream(k, s)) return check_launch(who);
     k.cw = cols_per_wg(a.N);
     const int64_t ng = (a.N + k.cw - 1) / k.cw;
     if (a.M <= 16) launch_mt<1>(k, ng, s);

@@ -53,6 +53,33 @@ def test_strided_x_and_errors():
         L.call("m2_skinny_gemm", a, 0)
 
 
+# The weight-streaming kernel (up to 16 rows): ends of K within a k step, a
+# unit of 64 and a wavefront's range, one to three column tiles with ragged
+# last ones, several rounds of workgroups, 8 and 16 wavefronts, padded row
+# strides.  |error| <= K 2^-24 sum |x w| bounds any order of a float32 sum of K
+# products.
+STREAM = [(1, 8, 1), (16, 64, 4), (3, 72, 700), (15, 1000, 4097), (16, 768, 12301), (2, 2568, 513),
+          (7, 3080, 8209), (9, 6144, 300), (16, 8192, 5000), (13, 8200, 77), (5, 1536, 24600)]
+
+
+@pytest.mark.parametrize("M,K,N", STREAM)
+def test_skinny_stream(M, K, N):
+    announce("skinny stream", M, K, N)
+    g = torch.Generator(device="cuda").manual_seed(M + 3 * K + N)
+    x = torch.randn((M, K + 24), generator=g, device="cuda").to(torch.bfloat16)[:, 8:8 + K]
+    w = torch.randn((N, K), generator=g, device="cuda").to(torch.bfloat16)
+    b = torch.randn(N, generator=g, device="cuda").to(torch.bfloat16)
+    y = linear_skinny(x, w, b, out_dtype=torch.float32)
+    ref = x.double() @ w.double().t() + b.double()
+    bound = (K + 1) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t() + b.double().abs())
+    err = (y.double() - ref).abs()
+    print(f"  max err / bound {float((err / bound).max()):.3f}", flush=True)
+    assert bool((err <= bound).all())
+    # rows past M and the columns of other workgroups are never written
+    z = linear_skinny(x[:1], w, b, out_dtype=torch.float32)
+    assert torch.equal(z[0], y[0])
+
+
 # ---------------------------------------------------------------------------
 # m2_skinny_gemm_norm: the rows normalised in the GEMM's prologue
 # ---------------------------------------------------------------------------
