@@ -6,7 +6,8 @@
 // per row and group of `group_size` consecutive elements.
 //
 // HBM-bound (x, z read once, out written once).  One workgroup per (row,
-// group): NT threads hold E chunks of CW elements each in registers (CW = 4:
+// group): NT threads (as the group and the number of groups ask, see the
+// launcher) hold E chunks of CW elements each in registers (CW = 4:
 // 16- / 8-byte accesses; CW = 1 for sizes that are not multiples of 4),
 // the sum of squares is reduced over the wavefronts in LDS, and the scaled
 // values are written from the registers.  Groups longer than NT * E are
@@ -161,10 +162,26 @@ int launch_rms_norm_gated(const m2_rms_norm_gated_args& a, hipStream_t s) {
     const dim3 grid((unsigned)nblocks);
     if (c4) {
         const int64_t n4 = a.group_size / 4;
-        if (n4 <= 64 * 4) hipLaunchKernelGGL((k_rms_norm<64, 4, 4>), grid, dim3(64), 0, s, k);
-        else if (n4 <= 256 * 2) hipLaunchKernelGGL((k_rms_norm<256, 2, 4>), grid, dim3(256), 0, s, k);
-        else if (n4 <= 256 * 4) hipLaunchKernelGGL((k_rms_norm<256, 4, 4>), grid, dim3(256), 0, s, k);
-        else hipLaunchKernelGGL((k_rms_norm<256, 8, 4>), grid, dim3(256), 0, s, k);
+        // Threads per (row, group), measured with a bf16 z or a residual, bf16 out
+        // (us before -> now).  Groups of up to 1024: one chunk per thread at every
+        // row count (768: 4.2 -> 3.1 at 16 rows, 10.3 -> 9.2 at 4096).  Up to one
+        // group per CU a workgroup's own latency is the time, so as many threads
+        // as there are chunks (16 rows: 2560 4.9 -> 4.0, 5120 7.0 -> 4.8, 8192 9.6
+        // -> 6.1).  More groups want fewer threads with two to four chunks in
+        // flight each (4096 rows: 5120 51.6 -> 39.4, 8192 93.6 -> 65.3, 4096 31.5 ->
+        // 30.6; one chunk per thread takes 41.2 / 67.1 / 36.2 there).
+        const bool few = nblocks <= cu_count();
+#define M2_NORM(NT, E) hipLaunchKernelGGL((k_rms_norm<NT, E, 4>), grid, dim3(NT), 0, s, k)
+        if (n4 <= 64) M2_NORM(64, 1);
+        else if (n4 <= 256) M2_NORM(256, 1);
+        else if (few && n4 <= 1024) M2_NORM(1024, 1);
+        else if (few && n4 <= 2048) M2_NORM(1024, 2);
+        else if (n4 <= 512) M2_NORM(256, 2);
+        else if (n4 <= 768) M2_NORM(256, 3);
+        else if (n4 <= 1024) M2_NORM(512, 2);
+        else if (n4 <= 2048) M2_NORM(512, 4);
+        else M2_NORM(1024, 4);
+#undef M2_NORM
     } else {
         if (a.group_size <= 64 * 8) hipLaunchKernelGGL((k_rms_norm<64, 8, 1>), grid, dim3(64), 0, s, k);
         else hipLaunchKernelGGL((k_rms_norm<256, 16, 1>), grid, dim3(256), 0, s, k);

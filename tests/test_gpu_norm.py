@@ -164,3 +164,20 @@ def _sweep_cases(n=20, seed=92):
 @pytest.mark.parametrize("case", _sweep_cases())
 def test_norm_sweep(case):
     test_norm_cases(case)
+
+
+@pytest.mark.parametrize("rows", [2, 300])
+@pytest.mark.parametrize("d", [256, 260, 1024, 1028, 2048, 2052, 3072, 3076, 4096, 4100, 8192, 8196, 16384, 16396])
+def test_threads_per_group(rows, d):
+    """The sizes at which the launcher changes the threads of a group, with fewer
+    and more rows than CUs: gate before the norm, and the residual add."""
+    announce("threads per group", rows, d)
+    rng = np.random.default_rng(rows + d)
+    x, z, res = (rng.standard_normal((rows, d)).astype(np.float32) for _ in range(3))
+    w = rng.uniform(0.5, 1.5, d).astype(np.float32)
+    want, _ = X.rms_norm_gated(x, w, z=z, norm_before_gate=False)
+    _close(rms_norm_gated(dev(x), dev(w), z=dev(z), norm_before_gate=False), want, False, "gated")
+    r = dev(res)
+    want, _ = X.rms_norm_gated(x + res, w)
+    _close(rms_norm_gated(dev(x), dev(w), residual=r), want, False, "residual")
+    assert np.array_equal(r.cpu().numpy(), x + res)
