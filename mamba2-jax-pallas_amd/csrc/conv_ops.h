@@ -45,20 +45,33 @@ struct UpdArgs {
     int silu;
 };
 
-// the conv output of channel c from its new state row s (already rounded to
-// the new state's dtype)
-template <int K> M2_DEV inline float conv_channel(const UpdArgs& a, const float (&s)[K], int64_t c) {
+// channel c's weights and bias
+template <int K> M2_DEV inline void conv_weights(const UpdArgs& a, int64_t c, float (&w)[K], float& bias) {
+#pragma unroll
+    for (int i = 0; i < K; ++i) w[i] = ldf(a.w, c * K + i, a.w_bf16);
+    bias = a.bias ? ldf(a.bias, c, a.bias_bf16) : 0.f;
+}
+
+// the conv output of a channel from its new state row s (already rounded to
+// the new state's dtype), its weights and bias
+template <int K>
+M2_DEV inline float conv_channel(const UpdArgs& a, const float (&s)[K], const float (&w)[K], float bias) {
     float acc = 0.f;
 #pragma unroll
     for (int i = 0; i < K; ++i) {
-        const float p = s[i] * ldf(a.w, c * K + i, a.w_bf16);
+        const float p = s[i] * w[i];
         acc += a.round_prod ? rbf(p) : p;
     }
     if (a.round_prod) acc = rbf(acc);
-    if (a.bias) acc += ldf(a.bias, c, a.bias_bf16);
+    if (a.bias) acc += bias;
     if (a.round_bias) acc = rbf(acc);
     if (a.silu) acc = silu_fast(acc);
     return acc;
+}
+template <int K> M2_DEV inline float conv_channel(const UpdArgs& a, const float (&s)[K], int64_t c) {
+    float w[K], bias;
+    conv_weights<K>(a, c, w, bias);
+    return conv_channel<K>(a, s, w, bias);
 }
 
 // output element (b, c) into the split output its channel belongs to
