@@ -215,6 +215,8 @@ int m2::ssd_combined_on(const m2_ssd_combined_args& a0, void* workspace, size_t 
     if (m2::ssd_walk_plan(a)) {
         // cumsum (+ weights) and CB in one launch, then the rest of the layer in
         // one kernel: their times land in the first and the last event interval
+        // (the slot of the weights, or that of the chunk states where the layout has
+        // no weights: head dim 32)
         float* wts = (float*)(ws + l.wts);
         if ((rc = m2::launch_ssd_walk_prep(a, dA, dto, wts, passed, s))) return rc;
         for (int i = 1; i < 5; ++i)

@@ -95,7 +95,7 @@ int launch_scan_fused(const m2_ssd_combined_args& a, const float* dA, const floa
 int ssd_combined_on(const m2_ssd_combined_args& a, void* ws, size_t ws_bytes, hipStream_t stream);
 
 // the whole combined forward in one chunk-sequential pass (csrc/ssd_walk.hip):
-// bf16, head dim 64, dstate 64 / 128 / 256, no seq_idx; its chunks are of 64
+// bf16, head dim 64 / 32, dstate 64 / 128 / 256, no seq_idx; its chunks are of 64
 // positions whatever chunk_size is.  launch_ssd_walk_prep computes chunk_cumsum's
 // dA / dt / weights for those and CB (in the workspace slot of the passed states,
 // which also holds the segment states of launch_ssd_walk behind it).

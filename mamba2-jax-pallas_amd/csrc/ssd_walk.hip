@@ -1,5 +1,5 @@
 // k_ssd_walk: chunk_state + state_passing + chunk_scan of the combined forward
-// in one pass for bf16 inputs (head dim 64, dstate 64 / 128 / 256).
+// in one pass for bf16 inputs (head dim 64 or 32, dstate 64 / 128 / 256).
 //
 //   y[m, :] = exp(dA[m]) C[m, :] bf16(h_c)^T                       (carried state)
 //           + sum_{k <= m} CB[m, k] exp(dA[m] - dA[k]) dt[k] x[k, :]  (intra chunk)
@@ -7,9 +7,9 @@
 //   h_{c+1} = exp(dA[last]) h_c + sum_q w[q] x[q, :]^T B[q, :]
 //
 // One workgroup walks the chunks (of 64 positions) of one chain -- a (batch,
-// head), all 64 head-dim rows or half of them -- with the running state in
-// MFMA accumulators, so neither the chunk states nor the states entering each
-// chunk pass through HBM: x, B, C and dt come in once and y goes out once.
+// head), all 64 head-dim rows, half of them, or a head of 32 -- with the running
+// state in MFMA accumulators, so neither the chunk states nor the states entering
+// each chunk pass through HBM: x, B, C and dt come in once and y goes out once.
 // CB = bf16(C B^T), shared by the heads of a group, is built ahead by k_walk_prep
 // in the register layout the walk reads.  Chains too few for the CUs are cut
 // into segments (k_seg_states gives each segment's end state from a zero start;
@@ -167,9 +167,9 @@ struct WalkArgs {
     const float* init;
     float* out;
     float* fin;
-    float* segst;          // [b, H, nseg - 1, 64, N]: each segment's end state from a zero start
+    float* segst;          // [b, H, nseg - 1, P, N]: each segment's end state from a zero start
     float* segdec;         // [b, H, nseg - 1]: its decay, prod exp(dA[last])
-    int L, H, G, nc, D_has_hdim, nwork;
+    int L, H, G, P, nc, D_has_hdim, nwork;
     int cps, nseg;         // chunks per segment, segments of a chain
 };
 
@@ -238,9 +238,9 @@ struct Loader {
 
     M2_DEV Loader(const WalkArgs& a, const char* ring, int bi, int h, int g, int p0, int li_, int lane_)
         : L(a.L), li(li_), lane(lane_) {
-        xs = a.x + ((int64_t)bi * a.L * a.H + h) * 64 + p0;
+        xs = a.x + ((int64_t)bi * a.L * a.H + h) * a.P + p0;
         bs = a.B + ((int64_t)bi * a.L * a.G + g) * S::N;
-        xst = (int64_t)a.H * 64;
+        xst = (int64_t)a.H * a.P;
         bst = (int64_t)a.G * S::N;
         auxp = (li == 0 ? a.dA : li == 1 ? a.dt : a.wts) + ((int64_t)bi * a.H + h) * a.nc * Q;
         ring_lds = lds_addr(ring);
@@ -305,8 +305,8 @@ struct StateTiles {
         for (int j = 0; j < NB8; ++j)
             bo[j] = XB + rA * BROW + (((n0 / 8 + 2 * j + (c4 >> 1)) ^ tswz<BROW>(rA)) * 16) + cb8;
     }
-    // offset of acc[0] in a [.., 64, N] state whose row p0 is the chain's first
-    M2_DEV int64_t off(int64_t bh, int p0) const { return (bh * 64 + p0 + prow) * N + n0 + 4 * kg; }
+    // offset of acc[0] in a [.., P, N] state whose row p0 is the chain's first
+    M2_DEV int64_t off(int64_t bh, int P, int p0) const { return (bh * P + p0 + prow) * N + n0 + 4 * kg; }
     M2_DEV void zero() {
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[j] = zero4();
@@ -427,7 +427,7 @@ M2_DEV void carry_path(const WalkArgs& a, const char* ring, const char* hs, char
 #pragma unroll
         for (int ns = 0; ns < NS; ++ns) r.c[ns] = *reinterpret_cast<const bf16x8*>(cp + 32 * ns);
         if constexpr (HASZ) {
-            const bf16* zp = a.z + ((b0 + row) * a.H + h) * 64 + p0 + 4 * kg;
+            const bf16* zp = a.z + ((b0 + row) * a.H + h) * a.P + p0 + 4 * kg;
 #pragma unroll
             for (int pt = 0; pt < PT; ++pt) r.z[pt] = *reinterpret_cast<const bf16x4*>(zp + 16 * pt);
         }
@@ -507,7 +507,7 @@ M2_DEV void intra_path(const WalkArgs& a, const char* ring, char* ys, float* ft,
         for (int q = 0; q < NPAIR; ++q) r.cb2[q] = *reinterpret_cast<const u32x4*>(cu + q * 512 + lane * 8);
         if constexpr (NU % 2 == 1) r.cb1 = *reinterpret_cast<const u32x2*>(cu + NPAIR * 512 + lane * 4);
         if constexpr (HASZ) {
-            const bf16* zp = a.z + ((b0 + min(c * Q + m, a.L - 1)) * a.H + h) * 64 + p0 + 4 * kg;
+            const bf16* zp = a.z + ((b0 + min(c * Q + m, a.L - 1)) * a.H + h) * a.P + p0 + 4 * kg;
 #pragma unroll
             for (int pt = 0; pt < PT; ++pt) r.z[pt] = *reinterpret_cast<const bf16x4*>(zp + 16 * pt);
         }
@@ -665,17 +665,17 @@ __global__ void __launch_bounds__(THREADS) k_ssd_walk(WalkArgs a) {
     __shared__ __align__(16) float ftab[4][64];
     __shared__ __align__(16) float Ds[64];
 
-    // work = ((batch nseg + segment) H + head) (64 / PW) + row part: the parts of a head and the
+    // work = ((batch nseg + segment) H + head) (P / PW) + row part: the parts of a head and the
     // heads of a group, which read the same x, B, C and CB, share an XCD
     const int work = xcd_remap(blockIdx.x, a.nwork);
-    constexpr int NPART = 64 / PW;
+    const int NPART = PT == 4 || a.P == PW ? 1 : 2;
     const int p0 = (work % NPART) * PW;
     const int bsh = work / NPART;
     const int h = bsh % a.H, seg = bsh / a.H % a.nseg, bi = bsh / a.H / a.nseg;
     const int g = h / (a.H / a.G);
     const int c0 = seg * a.cps, c1 = min(a.nc, c0 + a.cps);
     const int lane = threadIdx.x & 63, w = wave_id();
-    if (a.D && threadIdx.x < PW) Ds[threadIdx.x] = a.D_has_hdim ? a.D[h * 64 + p0 + threadIdx.x] : a.D[h];
+    if (a.D && threadIdx.x < PW) Ds[threadIdx.x] = a.D_has_hdim ? a.D[h * a.P + p0 + threadIdx.x] : a.D[h];
     __syncthreads();
 
     if (w < 4) {
@@ -699,12 +699,12 @@ __global__ void __launch_bounds__(THREADS) k_ssd_walk(WalkArgs a) {
         // y tiles staged between a chunk's barrier B and the next A.
         const int li = w - 12;
         constexpr int CPR = 4 * PT, RPS = 64 / CPR;          // 16-byte chunks per row, rows per store
-        float* ob = a.out + ((int64_t)bi * a.L * a.H + h) * 64 + p0;
+        float* ob = a.out + ((int64_t)bi * a.L * a.H + h) * a.P + p0;
         const int ch = lane % CPR, r0 = li * RPS + lane / CPR;   // rows r0 + ND RPS it
         constexpr int NIT = Q / RPS / ND, BT = NIT < 4 ? NIT : 4; // stores per chunk, per batch
         auto store = [&](int c) {
             const int valid = a.L - c * Q;
-            float* oc = ob + (int64_t)(c * Q + r0) * a.H * 64 + 4 * ch;
+            float* oc = ob + (int64_t)(c * Q + r0) * a.H * a.P + 4 * ch;
             // the reads of a batch first, so that their latencies overlap
 #pragma unroll
             for (int b = 0; b < NIT; b += BT) {
@@ -721,7 +721,7 @@ __global__ void __launch_bounds__(THREADS) k_ssd_walk(WalkArgs a) {
                 for (int q = 0; q < BT; ++q) {
                     const int m = r0 + ND * RPS * (b + q);
                     if (valid >= Q || m < valid)
-                        store_out<NTO>(u[q] + v[q], oc + (int64_t)(ND * RPS * (b + q)) * a.H * 64);
+                        store_out<NTO>(u[q] + v[q], oc + (int64_t)(ND * RPS * (b + q)) * a.H * a.P);
                 }
             }
         };
@@ -751,11 +751,11 @@ __global__ void __launch_bounds__(THREADS) k_ssd_walk(WalkArgs a) {
     // ---- the state wavefronts
     StateTiles<NS, PT> st(w - 8, lane);
     st.zero();
-    const int64_t bh64 = (int64_t)bi * a.H + h;
-    if (a.init) st.combine(a.init + st.off(bh64, p0), 0.f);
+    const int64_t bh = (int64_t)bi * a.H + h;
+    if (a.init) st.combine(a.init + st.off(bh, a.P, p0), 0.f);
     for (int i = 0; i < seg; ++i) {                          // the segments before this one
-        const int64_t o = bh64 * (a.nseg - 1) + i;
-        st.combine(a.segst + st.off(o, p0), a.segdec[o]);
+        const int64_t o = bh * (a.nseg - 1) + i;
+        st.combine(a.segst + st.off(o, a.P, p0), a.segdec[o]);
     }
     st.publish(hs + (S::DB ? (c0 & 1) * S::HS : 0));
     int k = 0;
@@ -767,7 +767,7 @@ __global__ void __launch_bounds__(THREADS) k_ssd_walk(WalkArgs a) {
         k = k + 1 == R ? 0 : k + 1;
     }
     lds_barrier();
-    if (a.fin && seg == a.nseg - 1) st.store(a.fin + st.off(bh64, p0));
+    if (a.fin && seg == a.nseg - 1) st.store(a.fin + st.off(bh, a.P, p0));
 }
 
 // ---------------------------------------------------------------------------
@@ -778,9 +778,9 @@ __global__ void __launch_bounds__(THREADS) k_ssd_walk(WalkArgs a) {
 // forming their state products) twice.  4 state and 4 data wavefronts, as in
 // the walk; one barrier per chunk.
 // ---------------------------------------------------------------------------
-template <int NS>
+template <int NS, int PT>
 __global__ void __launch_bounds__(512) k_seg_states(WalkArgs a) {
-    typedef WCfg<NS, 4> S;
+    typedef WCfg<NS, PT> S;
     constexpr int R = 3;
     __shared__ __align__(16) char ring[R * S::SLOT];
     const int work = xcd_remap(blockIdx.x, a.nwork);         // (b (nseg - 1) + segment) H + head
@@ -789,7 +789,7 @@ __global__ void __launch_bounds__(512) k_seg_states(WalkArgs a) {
     const int lane = threadIdx.x & 63, w = wave_id();
     if (w >= 4) {
         const int li = w - 4;
-        const Loader<NS, 4> ld(a, ring, bi, h, h / (a.H / a.G), 0, li, lane);
+        const Loader<NS, PT> ld(a, ring, bi, h, h / (a.H / a.G), 0, li, lane);
 #pragma unroll
         for (int i = 0; i < R - 1; ++i) ld.issue(min(c0 + i, c1 - 1), i);
         int k = R - 1;
@@ -803,7 +803,7 @@ __global__ void __launch_bounds__(512) k_seg_states(WalkArgs a) {
         wait_vmem<0>();
         return;
     }
-    StateTiles<NS, 4> st(w, lane);
+    StateTiles<NS, PT> st(w, lane);
     st.zero();
     float dec = 1.f;
     int k = 0;
@@ -813,7 +813,7 @@ __global__ void __launch_bounds__(512) k_seg_states(WalkArgs a) {
         k = k + 1 == R ? 0 : k + 1;
     }
     const int64_t o = ((int64_t)bi * a.H + h) * (a.nseg - 1) + seg;
-    st.store(a.segst + st.off(o, 0));
+    st.store(a.segst + st.off(o, a.P, 0));
     if (threadIdx.x == 0) a.segdec[o] = dec;
 }
 
@@ -839,7 +839,7 @@ struct WalkPlan {
 // whole, 266 halves).  Each round adds its start (first loads in flight), a
 // further segment its state's combination; the z gate a third of a step (128
 // heads, 4096 tokens: 123 us against 79).
-static double walk_cost(int64_t bh, int64_t nc, int64_t cps, int parts, int dstate, bool z, int64_t cus) {
+static double walk_cost(int64_t bh, int64_t nc, int64_t cps, int parts, bool half, int dstate, bool z, int64_t cus) {
     static const double step[3][2][2] = {{{0.68, 0.0029}, {0.57, 0.00125}},
                                          {{0.85, 0.0041}, {0.59, 0.0015}},
                                          {{1.70, 0.0032}, {1.20, 0.0031}}};
@@ -852,8 +852,8 @@ static double walk_cost(int64_t bh, int64_t nc, int64_t cps, int parts, int dsta
         const double st = f * (c0 + c1 * scale * (double)(r > 1 ? cap : wg));
         return r * (2.4 + cps * st * (r > 1 ? late : 1.0));
     };
-    const double* c = step[n][parts - 1];
-    double t = 8.0 + rounds(bh * nseg * parts, cus, z ? 1.3 : 1.0, c[0], c[1], parts == 2 ? 1.35 : 1.05);
+    const double* c = step[n][half ? 1 : 0];
+    double t = 8.0 + rounds(bh * nseg * parts, cus, z ? 1.3 : 1.0, c[0], c[1], half ? 1.35 : 1.05);
     if (nseg > 1)
         t += 4.0 + comb[n] * (double)(nseg - 1)
            + rounds(bh * (nseg - 1), n == 2 ? cus : 2 * cus, pre[n], 0.3, 0.0017, 1.0);
@@ -877,7 +877,7 @@ static double two_pass_cost(const m2_ssd_combined_args& a) {
 
 static WalkPlan walk_plan(const m2_ssd_combined_args& a) {
     const WalkPlan none{0, 0, 0};
-    if (a.dtype != M2_BF16 || a.headdim != 64 || a.seq_idx || a.varlen_states) return none;
+    if (a.dtype != M2_BF16 || (a.headdim != 64 && a.headdim != 32) || a.seq_idx || a.varlen_states) return none;
     if (a.dstate != 64 && a.dstate != 128 && a.dstate != 256) return none;
     if (a.ngroups <= 0 || a.nheads % a.ngroups || a.chunk_size % 64) return none;
     if (dispatch_override(M2_KNOB_STATES_SPLIT)) return none;
@@ -892,24 +892,28 @@ static WalkPlan walk_plan(const m2_ssd_combined_args& a) {
         return 2 * a.batch * nc * a.ngroups * CBU + 512 + 4 * bh * (nseg - 1) * (a.headdim * a.dstate + 1)
                <= 2 * bh * ncw * a.headdim * a.dstate;
     };
+    const bool p32 = a.headdim == 32;         // a whole head is what half of one of 64 is
     const int force = dispatch_override(M2_KNOB_LAYER);
     if (force == 3 || !fits(nc)) return none;
     if (force) {
         const int64_t seg = force >= 4 ? force / 2 : 1, cps = (nc + seg - 1) / seg;
         if (!fits(cps)) return none;
-        return {force >= 4 ? 1 + (force & 1) : force, cps, (nc + cps - 1) / cps};
+        return {p32 ? 1 : force >= 4 ? 1 + (force & 1) : force, cps, (nc + cps - 1) / cps};
     }
     WalkPlan best = none;
     double tb = 0.0;
-    for (int parts = 1; parts <= 2; ++parts)
+    for (int parts = 1; parts <= (p32 ? 1 : 2); ++parts)
         for (int64_t seg = 1; seg <= 32 && seg <= nc; ++seg) {
             const int64_t cps = (nc + seg - 1) / seg;
             // segments only where the chains leave CUs idle
             if (seg > 1 && (cps < 2 || !fits(cps) || bh * parts >= cu_count())) break;
-            const double t = walk_cost(bh, nc, cps, parts, (int)a.dstate, a.z != nullptr, cu_count());
+            const double t = walk_cost(bh, nc, cps, parts, p32 || parts == 2, (int)a.dstate, a.z != nullptr, cu_count());
             if (!best.parts || t < tb) { best = {parts, cps, (nc + cps - 1) / cps}; tb = t; }
         }
-    return tb < two_pass_cost(a) ? best : none;
+    // head dim 32 has no two-pass form, the other path is the five staged kernels:
+    // 4 x 6814 tokens of 10 heads 137 -> 45 us, 2 x 141 of 208 heads 61 -> 23, and no
+    // slower at any of 25 shapes
+    return p32 || tb < two_pass_cost(a) ? best : none;
 }
 
 int ssd_walk_plan(const m2_ssd_combined_args& a) {
@@ -956,23 +960,30 @@ int launch_ssd_walk(const m2_ssd_combined_args& a, const float* dA, const float*
     k.cb = (const bf16*)cb; k.dA = dA; k.dt = dt; k.wts = wts; k.D = a.D; k.init = a.initial_states;
     k.out = a.out; k.fin = a.final_states;
     k.L = (int)a.seqlen; k.H = (int)a.nheads; k.G = (int)a.ngroups;
-    k.nc = (int)((a.seqlen + Q - 1) / Q); k.D_has_hdim = a.D_has_hdim;
+    k.P = (int)a.headdim; k.nc = (int)((a.seqlen + Q - 1) / Q); k.D_has_hdim = a.D_has_hdim;
     k.cps = (int)p.cps; k.nseg = (int)p.nseg;
     const int64_t bh = a.batch * a.nheads, nwork = bh * p.nseg * p.parts;
     M2_REQUIRE(nwork < (1ll << 31), M2_ERR_UNSUPPORTED, "ssd_walk: too many workgroups");
     // behind CB, 256-byte aligned: the segment states, then their decays
     k.segst = (float*)((char*)cb + (2 * a.batch * k.nc * a.ngroups * CBU + 255) / 256 * 256);
-    k.segdec = k.segst + bh * (p.nseg - 1) * 64 * a.dstate;
+    k.segdec = k.segst + bh * (p.nseg - 1) * a.headdim * a.dstate;
     if (p.nseg > 1) {
         k.nwork = (int)(bh * (p.nseg - 1));
-        if (a.dstate == 64) k_seg_states<2><<<(unsigned)k.nwork, 512, 0, s>>>(k);
-        else if (a.dstate == 128) k_seg_states<4><<<(unsigned)k.nwork, 512, 0, s>>>(k);
-        else k_seg_states<8><<<(unsigned)k.nwork, 512, 0, s>>>(k);
+        const unsigned g = (unsigned)k.nwork;
+#define M2_SEG_L(NSV)                                                                      \
+    {                                                                                      \
+        if (k.P == 32) k_seg_states<NSV, 2><<<g, 512, 0, s>>>(k);                          \
+        else k_seg_states<NSV, 4><<<g, 512, 0, s>>>(k);                                    \
+    }
+        if (a.dstate == 64) M2_SEG_L(2)
+        else if (a.dstate == 128) M2_SEG_L(4)
+        else M2_SEG_L(8)
+#undef M2_SEG_L
     }
     k.nwork = (int)nwork;
     // outputs up to the 256 MB Infinity Cache are stored non-temporally (they
     // then do not evict the inputs still being read), as in k_scan_q128
-    const bool nt = (double)a.batch * a.seqlen * a.nheads * 64 * 4 <= 256.0 * (1 << 20);
+    const bool nt = (double)a.batch * a.seqlen * a.nheads * a.headdim * 4 <= 256.0 * (1 << 20);
 #define M2_WALK_L(NSV, PTV, ZV)                                                            \
     {                                                                                      \
         if (nt) k_ssd_walk<NSV, PTV, ZV, true><<<(unsigned)nwork, THREADS, 0, s>>>(k);     \
@@ -980,7 +991,7 @@ int launch_ssd_walk(const m2_ssd_combined_args& a, const float* dA, const float*
     }
 #define M2_WALK_P(NSV)                                                                     \
     {                                                                                      \
-        if (p.parts == 1) { if (a.z) M2_WALK_L(NSV, 4, true) else M2_WALK_L(NSV, 4, false) } \
+        if (p.parts == 1 && k.P == 64) { if (a.z) M2_WALK_L(NSV, 4, true) else M2_WALK_L(NSV, 4, false) } \
         else { if (a.z) M2_WALK_L(NSV, 2, true) else M2_WALK_L(NSV, 2, false) }            \
     }
     if (a.dstate == 64) M2_WALK_P(2)

@@ -20,7 +20,7 @@ from oracle import ssd_oracle as O
 pytestmark = pytest.mark.gpu
 
 PLANS = ["walk", "walk_half", "walk_x2", "walk_half_x3", "walk_x32"]
-# (batch, L, H, G, dstate, chunk, init, z, D per head dim)
+# (batch, L, H, G, dstate, chunk, init, z, D per head dim[, head dim])
 SHAPES = [
     (1, 1, 2, 1, 128, 128, False, False, False),
     (2, 63, 4, 2, 64, 64, True, False, True),
@@ -30,14 +30,17 @@ SHAPES = [
     (1, 447, 4, 1, 256, 64, False, False, True),
     (1, 1000, 5, 1, 64, 128, True, True, True),
     (2, 1088, 4, 4, 128, 256, True, False, False),
+    (1, 65, 4, 2, 128, 256, True, True, False, 32),
+    (2, 700, 6, 1, 64, 128, False, False, True, 32),
+    (1, 1000, 4, 1, 256, 64, True, False, False, 32),
 ]
 
 
-def _inputs(b, Lq, H, G, N, Q, init, z, dhp, seed):
-    cfg = configs.SSDConfig("walk", b, Lq, H, G, 64, N, Q, "bf16", init_state=init, seed=seed)
+def _inputs(b, Lq, H, G, N, Q, init, z, dhp, P=64, *, seed):
+    cfg = configs.SSDConfig("walk", b, Lq, H, G, P, N, Q, "bf16", init_state=init, seed=seed)
     d = configs.make_ssd_inputs(cfg, with_z=z)
     if dhp:
-        d["D"] = np.random.default_rng(seed).uniform(0.5, 1.5, (H, 64)).astype(np.float32)
+        d["D"] = np.random.default_rng(seed).uniform(0.5, 1.5, (H, P)).astype(np.float32)
     d.pop("seq_idx"), d.pop("cu_seqlens")
     T = tdtype("bf16")
     t = {k: dev(v, T if k in ("x", "dt", "B", "C", "z") else None) for k, v in d.items()}
