@@ -34,7 +34,7 @@
 // CB that each workgroup reads from L2 are 37 of its 42 KB.  The layer at 128
 // heads, dstate 128, 4096 tokens takes 79 us (2.7 TB/s over its compulsory 223
 // MB) against 107 for the state pass and the scan, at 256 heads, dstate 256, 182
-// against 276, at 24 heads and 30011 tokens 147 against 364 in 10 segments.
+// against 276, at 24 heads and 30011 tokens 143 against 364 in 10 segments.
 // Chunks of 128 would halve the barriers, but their operands do not fit LDS
 // twice at dstate 256.  One wavefront for carry and intra together: 93 against
 // 82 us at the first shape; loads issued by two wavefronts: 100.
@@ -185,8 +185,10 @@ struct WCfg {
     static constexpr int YT = Q * PW * 4, YS = 2 * YT;       // staged y tiles: carried, intra
     static constexpr int FT = 4 * 64 * 4;                    // decay factors per y wavefront
     // double-buffered state and y tiles (one barrier per chunk) where a ring of
-    // three slots still fits beside them
-    static constexpr bool DB = 3 * SLOT + 2 * (HS + YS) + FT + 256 <= LDS_BYTES;
+    // two slots still fits beside them: at dstate 128 a whole head with two
+    // barriers and three slots took 107 us (128 heads, 4096 tokens) against 98, at
+    // dstate 256 halves (256 heads) 282 against 261
+    static constexpr bool DB = 2 * SLOT + 2 * (HS + YS) + FT + 256 <= LDS_BYTES;
     static constexpr int NBUF = DB ? 2 : 1;
     static constexpr int FIXED = NBUF * (HS + YS) + FT + 256;
     static constexpr int R = 4 * SLOT + FIXED <= LDS_BYTES ? 4 : 3 * SLOT + FIXED <= LDS_BYTES ? 3 : 2;
@@ -730,10 +732,14 @@ __global__ void __launch_bounds__(THREADS) k_ssd_walk(WalkArgs a) {
         for (int i = 0; i < R - 1; ++i) ld.issue(min(c0 + i, c1 - 1), i);
         int k = R - 1;                                       // the slot of chunk c + R - 1
         for (int c = c0; c < c1; ++c) {
-            // the loads of chunk c done (later ones may be in flight; the stores
-            // issued in between only make the wait longer)
-            if (li < 3) wait_vmem<S::WAIT0>();
-            else wait_vmem<S::WAIT1>();
+            // the loads of chunk c done: vmcnt counts down in issue order, and
+            // behind them came the loads of R - 2 chunks and, from the R-th chunk
+            // on, the NIT stores of R - 1 (all of them full chunks: the last one's
+            // follow the loop).  Not waiting for the stores too is worth 3 % with a
+            // ring of two (128 whole heads at dstate 128: 101 -> 98 us)
+            if (c < c0 + R) wait_vmem<S::WAIT1>();
+            else if (li < 3) wait_vmem<S::WAIT0 + (R - 1) * NIT>();
+            else wait_vmem<S::WAIT1 + (R - 1) * NIT>();
             lds_barrier();                                   // A: chunk c's slot complete, chunk c - 1's free
             // between A and B, where the other wavefronts compute: between B and A
             // they would wait for it
