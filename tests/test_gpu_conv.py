@@ -139,6 +139,22 @@ def test_conv_paths(case):
     _close(got, want, rdt == "bfloat16", f"{layout} k={k}", _mag(x, w, bias))
 
 
+@pytest.mark.parametrize("L", [1, 15, 16, 17, 31, 64, 79])
+@pytest.mark.parametrize("k,dt", [(4, "bf16"), (6, "bf16"), (7, "bf16"), (8, "f32")])
+def test_conv_runs(L, k, dt):
+    """Channels-last runs of 16 tokens: lengths around a whole run and a whole
+    workgroup of them, widths on both sides of the unrolled form."""
+    announce("causal_conv1d runs", L, k, dt)
+    rng = np.random.default_rng(100 * L + k)
+    t = {"bf16": torch.bfloat16, "f32": torch.float32}[dt]
+    x, w, bias = _inputs(rng, 2, 520, L, k, t, t, t)
+    for seq in (None, _seq(rng, 2, L, 3) if L > 1 else None):
+        want, rdt = X.causal_conv1d(x, w, bias, "silu", seq, NAME[t], NAME[t], NAME[t])
+        got = causal_conv1d(_layout(dev(x, t), "cl"), dev(w, t), dev(bias, t), "silu",
+                            None if seq is None else dev(seq))
+        _close(got, want, rdt == "bfloat16", f"L={L} k={k}", _mag(x, w, bias))
+
+
 def test_conv_weight_3d_and_unaligned():
     rng = np.random.default_rng(3)
     x, w, bias = _inputs(rng, 1, 16, 33, 4, None, None, None)
