@@ -216,11 +216,13 @@ def scan_is_fused(cfg, states_fused=None):
             and cfg.chunk_size in (64, 128))
 
 
-def measured_traffic(config):
+def measured_traffic(config, dom=None):
     """HBM bytes per launch of each stage as measured by rocprofv3 FETCH_SIZE /
     WRITE_SIZE (scaled by a plain copy's readings) for this config, from
-    profiles/hbm_traffic_<config>.json; empty when there is none."""
-    path = os.path.join(ROOT, "profiles", f"hbm_traffic_{config}.json")
+    profiles/hbm_traffic_<config>.json (hbm_traffic_walk_<config>.json where the
+    dominant stage `dom` is one of the one-pass walk's); empty when there is none."""
+    walk = "walk_" if dom in (WALK_PREP, WALK) else ""
+    path = os.path.join(ROOT, "profiles", f"hbm_traffic_{walk}{config}.json")
     if not os.path.exists(path):
         return {}
     with open(path) as f:
@@ -682,7 +684,7 @@ def bench_other_config(name, steps=200, warmup=20, cpu=True):
     finish = stage_table_enqueue(cfg, kw, nev, stage_events(cfg, nev, layer_plan(cfg, kw)))
     ms, _ = time_layer(kw, steps, warmup)
     stages, dom, roof, _, tot_by = finish()
-    attach_traffic(roof, measured_traffic(name), dom)
+    attach_traffic(roof, measured_traffic(name, dom), dom)
     out = {"workload": f"{cfg.name} SSD layer forward ({name})", "dtype": cfg.dtype,
            "batch": cfg.batch, "seq_len": cfg.seqlen, "nheads": cfg.nheads,
            "ngroups": cfg.ngroups, "headdim": cfg.headdim, "dstate": cfg.dstate,
@@ -786,7 +788,7 @@ def main(argv=None):
     ms, wall_ms = time_layer(kw, K, args.warmup)
     stages, dom, roof, stages_ms_total, tot_by = finish()
     # measured traffic is kept for each config at its own dtype
-    attach_traffic(roof, measured_traffic(args.config) if own_dtype else {}, dom)
+    attach_traffic(roof, measured_traffic(args.config, dom) if own_dtype else {}, dom)
     res = {
         "metric": METRIC, "value": cfg.tokens / (ms * 1e-3), "unit": "tokens/s",
         "n_gpus": 1, "steps": K, "warmup": args.warmup, "ms_per_step": ms,

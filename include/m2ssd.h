@@ -214,7 +214,10 @@ typedef struct {
                                        NULL entry is not recorded.  With bf16
                                        and the fused scan the varlen states
                                        run after state_passing, so event 6
-                                       is recorded before events 4 and 5    */
+                                       is recorded before events 4 and 5.  On
+                                       the one-pass path everything before the
+                                       walk ends at event 1 and the walk at
+                                       event 5; events 2-4 come with event 1 */
 } m2_ssd_combined_args;
 size_t m2_ssd_combined_workspace_size(const m2_ssd_combined_args* a);
 

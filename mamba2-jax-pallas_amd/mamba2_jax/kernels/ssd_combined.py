@@ -3,12 +3,13 @@
 Drop-in for reference kernels/ssd_combined.py:46-203, for every head dim and
 dstate (sizes the kernels do not tile run through the exact padding / head
 splitting / dstate blocks of kernels/_shapes.py).  One call into
-libm2ssd.so (m2_ssd_combined) enqueues the five stage kernels
-(chunk_cumsum -> chunk_state -> state_passing -> bmm_chunk -> chunk_scan, plus
-chunk_state_varlen when varlen states are requested) on the current stream;
-the intermediates live in a workspace drawn from torch's caching allocator.
-As in the reference, the state entering each chunk is kept in x's dtype,
-while the output and the final states are float32.
+libm2ssd.so (m2_ssd_combined) enqueues the five stages on the current stream:
+chunk_cumsum -> chunk_state -> state_passing -> bmm_chunk -> chunk_scan (plus
+chunk_state_varlen when varlen states are requested) as separate or fused
+kernels, or, for bf16 at the sizes it is built for, a prologue and one walk over
+each chain.  The intermediates live in a workspace drawn from torch's caching
+allocator.  As in the reference, the state entering each chunk is rounded to
+x's dtype, while the output and the final states are float32.
 """
 
 from __future__ import annotations

@@ -14,9 +14,9 @@ from .. import _lib as L
 
 MAX_ROWS = 64
 # rows up to which the decode path uses the skinny kernel (measured on MI355X
-# in the 2.7b-shape decode graph at batch 1: in-projection 22 -> 15.9 us,
-# out-projection 17 -> 10.5 us per layer; at 64 rows hipBLASLt's tiles are
-# faster)
+# in the 2.7b-shape decode: in-projection 22 us with hipBLASLt, 12.2 with the
+# weights streamed through LDS, out-projection 17 and 8.5; at 64 rows
+# hipBLASLt's tiles are faster)
 PREFERRED_ROWS = 16
 
 
