@@ -216,19 +216,24 @@ M2_DEV void dma4(const void* g, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
                  ::"s"(__builtin_amdgcn_readfirstlane(lds)), "v"(g) : "memory", "m0");
 }
-// the same from a scalar base (uniform over the wavefront) plus a per-lane byte
-// offset: no vector address arithmetic per load
+// The same from a scalar base (uniform over the wavefront) plus a per-lane byte
+// offset: no vector address arithmetic per load.  A vector memory instruction
+// that reads a scalar register needs five wait states behind the vector
+// instruction that wrote it; the compiler, which keeps them for its own loads,
+// cannot see this one, and uniform_ptr's v_readfirstlane may stand right before it
+// (it did in k_seg_states at dstate 128 and 256).  The M0 write and s_nop 3 are
+// five, whatever the compiler puts in front.
 M2_DEV const void* uniform_ptr(const void* g) {
     const uint64_t v = (uint64_t)g;
     return (const void*)(((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(v >> 32)) << 32) |
                          (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)v));
 }
 M2_DEV void dma16s(const void* base, uint32_t off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2"
                  ::"s"(__builtin_amdgcn_readfirstlane(lds)), "v"(off), "s"(uniform_ptr(base)) : "memory", "m0");
 }
 M2_DEV void dma4s(const void* base, uint32_t off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dword %1, %2"
                  ::"s"(__builtin_amdgcn_readfirstlane(lds)), "v"(off), "s"(uniform_ptr(base)) : "memory", "m0");
 }
 #pragma clang diagnostic pop

@@ -240,11 +240,12 @@ struct Loader {
 
     M2_DEV Loader(const WalkArgs& a, const char* ring, int bi, int h, int g, int p0, int li_, int lane_)
         : L(a.L), li(li_), lane(lane_) {
-        xs = a.x + ((int64_t)bi * a.L * a.H + h) * a.P + p0;
-        bs = a.B + ((int64_t)bi * a.L * a.G + g) * S::N;
+        // scalar from here on, so that a load's base needs no v_readfirstlane
+        xs = (const bf16*)uniform_ptr(a.x + ((int64_t)bi * a.L * a.H + h) * a.P + p0);
+        bs = (const bf16*)uniform_ptr(a.B + ((int64_t)bi * a.L * a.G + g) * S::N);
         xst = (int64_t)a.H * a.P;
         bst = (int64_t)a.G * S::N;
-        auxp = (li == 0 ? a.dA : li == 1 ? a.dt : a.wts) + ((int64_t)bi * a.H + h) * a.nc * Q;
+        auxp = (const float*)uniform_ptr((li == 0 ? a.dA : li == 1 ? a.dt : a.wts) + ((int64_t)bi * a.H + h) * a.nc * Q);
         ring_lds = lds_addr(ring);
         xv = 2 * (uint32_t)(lane / S::XCPR * xst + ((lane % S::XCPR) ^ tswz<XROW>(lane / S::XCPR)) * 8);
 #pragma unroll
