@@ -177,8 +177,10 @@ int m2_chunk_state_varlen(const m2_chunk_state_varlen_args* a, void* stream);
  * bmm_chunk -> chunk_scan [-> varlen states]) on one stream, intermediates in
  * the caller's workspace (size from m2_ssd_combined_workspace_size).
  * states_passed is kept in x's dtype; out and the final states are float32.
- * chunk_size is a tiling choice here as in the reference (the outputs are the
- * same function of the inputs for every chunk size): any positive chunk size
+ * chunk_size is a tiling choice here as in the reference (with A <= 0 and
+ * dt' >= 0 the outputs are the same function of the inputs for every chunk size;
+ * else the states' decay exp(min(dA_last - dA, 0)) is clamped chunk by chunk):
+ * any positive chunk size
  * is accepted; bf16 chunk sizes the fused kernels do not take run as chunks of
  * 128 when that keeps the whole layer on the fused kernels, fp32 chunks of 256
  * and chunk sizes other than 64 / 128 / 256 run as chunks of 128.  Head dim

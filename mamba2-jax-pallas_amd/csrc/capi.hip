@@ -139,8 +139,10 @@ int record(void** ev, int i, hipStream_t s) {
 }
 
 // The combined forward returns only y and the final (and varlen) states: the
-// same function of the inputs for every chunk size (the chunked algorithm is
-// exact; only the rounding points at chunk boundaries move).  bf16 chunk
+// same function of the inputs for every chunk size where dA falls (A <= 0 and
+// dt' >= 0; the chunked algorithm is exact and only the rounding points at chunk
+// boundaries move).  Where it rises, the clamp of the chunk states' decay makes
+// the states depend on the chunk size chosen here, on every path alike.  bf16 chunk
 // sizes the fused kernels do not take (256: the fused scan keeps at most 128
 // positions of a chunk in LDS; 32; ...) run as chunks of 128 when that puts
 // both halves of the layer on the fused kernels; fp32 chunks of 256 always

@@ -40,6 +40,7 @@
 // 82 us at the first shape; loads issued by two wavefronts: 100.
 //
 // Follows reference ops/ssd_naive.py:189-318 (chunk_scan), :77-182 (states).
+#include <cfloat>
 #include <type_traits>
 
 #include "cumsum_tile.h"
@@ -163,6 +164,7 @@ struct WalkArgs {
     const float* dA;       // [b, H, nc, Q]
     const float* dt;
     const float* wts;
+    const float* A;        // [H]
     const float* D;
     const float* init;
     float* out;
@@ -171,7 +173,20 @@ struct WalkArgs {
     float* segdec;         // [b, H, nseg - 1]: its decay, prod exp(dA[last])
     int L, H, G, P, nc, D_has_hdim, nwork;
     int cps, nseg;         // chunks per segment, segments of a chain
+    int sub;               // the walk's chunks in one of the layer's (cps: a multiple, if nseg > 1)
 };
+
+// A > 0 (dA rises): the layer's state weights exp(min(dA[last] - dA, 0)) dt are
+// clamped over its own chunks of `sub` of the walk's, while its output is not.
+// The state wavefronts of such a head (RISING below) keep two states: the layer's, with
+// those weights, and one without the clamp for the outputs inside a chunk.
+M2_DEV bool rising(const WalkArgs& a, int h) { return a.sub > 1 && a.A[h] > 0.f; }
+// dA over the layer's chunk that starts at the walk's chunk c (dl: the chain's dA[last])
+M2_DEV float chunk_total(const float* dl, int c, int sub, int nc) {
+    float t = 0.f;
+    for (int i = c; i < min(c + sub, nc); ++i) t += dl[(int64_t)i * Q];
+    return t;
+}
 
 template <int NS, int PT>
 struct WCfg {
@@ -331,11 +346,12 @@ struct StateTiles {
     // the bf16 state into LDS rows [PW][N]
     M2_DEV void publish(char* hs) const {
 #pragma unroll
-        for (int j = 0; j < NT; ++j) {
-            const int n = n0 + 16 * j + 4 * kg;
-            const u32x2 p = {pk_bf16(acc[j][0], acc[j][1]), pk_bf16(acc[j][2], acc[j][3])};
-            *reinterpret_cast<u32x2*>(hs + prow * (2 * N) + (((n >> 3) ^ sswz<S::BCPR>(prow)) * 16) + 2 * (n & 7)) = p;
-        }
+        for (int j = 0; j < NT; ++j) publish(j, acc[j], hs);
+    }
+    M2_DEV void publish(int j, const f32x4& v, char* hs) const {
+        const int n = n0 + 16 * j + 4 * kg;
+        const u32x2 p = {pk_bf16(v[0], v[1]), pk_bf16(v[2], v[3])};
+        *reinterpret_cast<u32x2*>(hs + prow * (2 * N) + (((n >> 3) ^ sswz<S::BCPR>(prow)) * 16) + 2 * (n & 7)) = p;
     }
     // h <- exp(dA[last]) h + B^T (w x) over the chunk in `slot`; returns exp(dA[last])
     M2_DEV float step(const char* slot) {
@@ -403,6 +419,61 @@ struct StateTiles {
             }
         }
         return sc;
+    }
+    // The same for a rising chain, a tile at a time (a second state may be live):
+    // out(j, h_j f + B^T (w x)), w = exp(expo(dA)) dt.
+    template <typename E, typename O>
+    M2_DEV void tiles(const f32x4 (&h)[NT], const char* slot, float f, E expo, O out) const {
+        const float* aux = reinterpret_cast<const float*>(slot + XB + BB);
+        bf16x8 xh[2], xl[2];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            uint32_t hi[4], lo[4];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int q = 32 * ks + 16 * i;
+                const float4 d = *reinterpret_cast<const float4*>(aux + q + 4 * kg);
+                const float4 t = *reinterpret_cast<const float4*>(aux + Q + q + 4 * kg);
+                const u32x2 p = __builtin_bit_cast(u32x2, ds_read_tr(slot + xo0 + q * XROW));
+                split2(bf16_lo(p[0]) * (ex2(expo(d.x) * LOG2E) * t.x), bf16_hi(p[0]) * (ex2(expo(d.y) * LOG2E) * t.y),
+                       hi[2 * i], lo[2 * i]);
+                split2(bf16_lo(p[1]) * (ex2(expo(d.z) * LOG2E) * t.z), bf16_hi(p[1]) * (ex2(expo(d.w) * LOG2E) * t.w),
+                       hi[2 * i + 1], lo[2 * i + 1]);
+            }
+            xh[ks] = as_bf16x8(hi[0], hi[1], hi[2], hi[3]);
+            xl[ks] = as_bf16x8(lo[0], lo[1], lo[2], lo[3]);
+        }
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            __builtin_amdgcn_sched_barrier(0);
+            const int o = bo[j % NB8] + (j / 8) * 256;
+            f32x4 v = h[j];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] *= f;
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                const bf16x4 ba = ds_read_tr(slot + o + 32 * ks * BROW);
+                const bf16x4 bb = ds_read_tr(slot + o + (32 * ks + 16) * BROW);
+                const bf16x8 bf = __builtin_shufflevector(ba, bb, 0, 1, 2, 3, 4, 5, 6, 7);
+                v = mma32(bf, xh[ks], v);
+                v = mma32(bf, xl[ks], v);
+            }
+            out(j, v);
+        }
+    }
+    // the layer's state: total, the dA of the layer's chunk; before, that of its
+    // earlier chunks of the walk.  The state takes all of the factor exp(total)
+    // (returned) with the layer's chunk's first
+    M2_DEV float step_clamped(const char* slot, float total, float before, bool first) {
+        const float f = first ? ex2(total * LOG2E) : 1.f;
+        tiles(acc, slot, f, [&](float d) { return fminf(total - (d + before), 0.f); },
+              [&](int j, const f32x4& v) { acc[j] = v; });
+        return f;
+    }
+    // the unclamped state behind h
+    template <typename O> M2_DEV void step_free(const f32x4 (&h)[NT], const char* slot, O out) const {
+        const float dl = reinterpret_cast<const float*>(slot + XB + BB)[Q - 1];
+        tiles(h, slot, ex2(dl * LOG2E), [&](float d) { return dl - d; }, out);
     }
 };
 
@@ -658,6 +729,75 @@ M2_DEV void intra_path(const WalkArgs& a, const char* ring, char* ys, float* ft,
     lds_barrier();                                           // the last chunk's y staged
 }
 
+// ---- a state wavefront: h_{c+1} from chunk c, published in bf16 for the carry
+// wavefronts.
+template <int NS, int PT, bool RISING>
+M2_DEV void state_path(const WalkArgs& a, const char* ring, char* hs, int sw, int bi, int h, int seg, int p0, int c0, int c1) {
+    typedef WCfg<NS, PT> S;
+    constexpr int R = S::R, SLOT = S::SLOT;
+    int lane = threadIdx.x & 63;
+    // keeps the rare path's address registers its own, not live beside the other's
+    if constexpr (RISING) asm volatile("" : "+v"(lane));
+    StateTiles<NS, PT> st(sw, lane);
+    st.zero();
+    const int64_t bh = (int64_t)bi * a.H + h;
+    if (a.init) st.combine(a.init + st.off(bh, a.P, p0), 0.f);
+    for (int i = 0; i < seg; ++i) {                          // the segments before this one
+        const int64_t o = bh * (a.nseg - 1) + i;
+        st.combine(a.segst + st.off(o, a.P, p0), a.segdec[o]);
+    }
+    st.publish(hs + (S::DB ? (c0 & 1) * S::HS : 0));
+    int k = 0;
+    if constexpr (!RISING) {
+        for (int c = c0; c < c1; ++c) {
+            lds_barrier();                                   // A
+            st.step(ring + k * SLOT);
+            if constexpr (!S::DB) lds_barrier();             // B
+            st.publish(hs + (S::DB ? ((c + 1) & 1) * S::HS : 0));    // h_{c+1}
+            k = k + 1 == R ? 0 : k + 1;
+        }
+    } else {
+        // st: the layer's state (c0 starts a chunk of the layer); free: the unclamped
+        // one, needed for more than the next chunk only where a chunk of the layer is
+        // more than two of the walk's (head dim 32)
+        constexpr bool KEEP = PT == 2;
+        const float* dl = a.dA + bh * a.nc * Q + Q - 1;
+        // before each publish: its addresses are formed anew, kept they would spill
+        auto fresh = [&]() { asm volatile("" : "+v"(st.prow), "+v"(KEEP ? st.n0 : st.kg)); };
+        f32x4 free[S::NT];
+        float total = 0.f, before = 0.f;
+        for (int c = c0; c < c1; ++c) {
+            const bool first = c % a.sub == 0, last = (c + 1) % a.sub == 0;
+            const char* slot = ring + k * SLOT;
+            char* const hn = hs + (S::DB ? ((c + 1) & 1) * S::HS : 0);
+            if (first) {
+                total = chunk_total(dl, c, a.sub, a.nc);
+                before = 0.f;
+                if constexpr (KEEP) {
+#pragma unroll
+                    for (int j = 0; j < S::NT; ++j) free[j] = st.acc[j];
+                }
+            }
+            lds_barrier();                                   // A
+            if constexpr (!S::DB) lds_barrier();             // B: slots change hands at A only
+            if (!last) {
+                fresh();
+                if constexpr (KEEP) st.step_free(free, slot, [&](int j, const f32x4& v) { free[j] = v; st.publish(j, v, hn); });
+                else st.step_free(st.acc, slot, [&](int j, const f32x4& v) { st.publish(j, v, hn); });
+            }
+            st.step_clamped(slot, total, before, first);
+            if (last) {
+                fresh();
+                st.publish(hn);
+            }
+            before += dl[(int64_t)c * Q];
+            k = k + 1 == R ? 0 : k + 1;
+        }
+    }
+    lds_barrier();
+    if (a.fin && seg == a.nseg - 1) st.store(a.fin + st.off(bh, a.P, p0));
+}
+
 template <int NS, int PT, bool HASZ, bool NTO>
 __global__ void __launch_bounds__(THREADS) k_ssd_walk(WalkArgs a) {
     typedef WCfg<NS, PT> S;
@@ -756,25 +896,8 @@ __global__ void __launch_bounds__(THREADS) k_ssd_walk(WalkArgs a) {
     }
 
     // ---- the state wavefronts
-    StateTiles<NS, PT> st(w - 8, lane);
-    st.zero();
-    const int64_t bh = (int64_t)bi * a.H + h;
-    if (a.init) st.combine(a.init + st.off(bh, a.P, p0), 0.f);
-    for (int i = 0; i < seg; ++i) {                          // the segments before this one
-        const int64_t o = bh * (a.nseg - 1) + i;
-        st.combine(a.segst + st.off(o, a.P, p0), a.segdec[o]);
-    }
-    st.publish(hs + (S::DB ? (c0 & 1) * S::HS : 0));
-    int k = 0;
-    for (int c = c0; c < c1; ++c) {
-        lds_barrier();                                       // A
-        st.step(ring + k * SLOT);
-        if constexpr (!S::DB) lds_barrier();                 // B
-        st.publish(hs + (S::DB ? ((c + 1) & 1) * S::HS : 0));    // h_{c+1}
-        k = k + 1 == R ? 0 : k + 1;
-    }
-    lds_barrier();
-    if (a.fin && seg == a.nseg - 1) st.store(a.fin + st.off(bh, a.P, p0));
+    if (rising(a, h)) state_path<NS, PT, true>(a, ring, hs, w - 8, bi, h, seg, p0, c0, c1);
+    else state_path<NS, PT, false>(a, ring, hs, w - 8, bi, h, seg, p0, c0, c1);
 }
 
 // ---------------------------------------------------------------------------
@@ -812,14 +935,30 @@ __global__ void __launch_bounds__(512) k_seg_states(WalkArgs a) {
     }
     StateTiles<NS, PT> st(w, lane);
     st.zero();
+    const int64_t bh = (int64_t)bi * a.H + h;
     float dec = 1.f;
     int k = 0;
-    for (int c = c0; c < c1; ++c) {
-        lds_barrier();
-        dec *= st.step(ring + k * S::SLOT);
-        k = k + 1 == R ? 0 : k + 1;
+    if (rising(a, h)) {
+        const float* dl = a.dA + bh * a.nc * Q + Q - 1;
+        float total = 0.f, before = 0.f;
+        for (int c = c0; c < c1; ++c) {
+            const bool first = c % a.sub == 0;
+            if (first) { total = chunk_total(dl, c, a.sub, a.nc); before = 0.f; }
+            lds_barrier();
+            dec *= st.step_clamped(ring + k * S::SLOT, total, before, first);
+            before += dl[(int64_t)c * Q];
+            k = k + 1 == R ? 0 : k + 1;
+        }
+        // an overflowing factor must not turn a zero state into NaN
+        dec = fminf(dec, FLT_MAX);
+    } else {
+        for (int c = c0; c < c1; ++c) {
+            lds_barrier();
+            dec *= st.step(ring + k * S::SLOT);
+            k = k + 1 == R ? 0 : k + 1;
+        }
     }
-    const int64_t o = ((int64_t)bi * a.H + h) * (a.nseg - 1) + seg;
+    const int64_t o = bh * (a.nseg - 1) + seg;
     st.store(a.segst + st.off(o, a.P, 0));
     if (threadIdx.x == 0) a.segdec[o] = dec;
 }
@@ -886,10 +1025,11 @@ static WalkPlan walk_plan(const m2_ssd_combined_args& a) {
     const WalkPlan none{0, 0, 0};
     if (a.dtype != M2_BF16 || (a.headdim != 64 && a.headdim != 32) || a.seq_idx || a.varlen_states) return none;
     if (a.dstate != 64 && a.dstate != 128 && a.dstate != 256) return none;
-    if (a.ngroups <= 0 || a.nheads % a.ngroups || a.chunk_size % 64) return none;
+    if (a.ngroups <= 0 || a.nheads % a.ngroups || a.chunk_size % Q) return none;
+    if (a.headdim == 64 && a.chunk_size > 2 * Q) return none;       // state_path's rising chains
     if (dispatch_override(M2_KNOB_STATES_SPLIT)) return none;
-    // dt' >= 0, so that dA is monotonic within a chunk: the chunk states' decay is
-    // clamped at 0, which depends on the chunk size where dA both rises and falls
+    // dt' >= 0, so that dA is monotonic: the intra-chunk weights' two factors need
+    // it, and it leaves the clamp of the state weights to the sign of A (rising())
     if (!(a.dt_max >= 0.f && (a.dt_softplus || a.dt_min >= 0.f))) return none;
     const int64_t nc = (a.seqlen + Q - 1) / Q, ncw = (a.seqlen + a.chunk_size - 1) / a.chunk_size;
     const int64_t bh = a.batch * a.nheads;
@@ -900,10 +1040,13 @@ static WalkPlan walk_plan(const m2_ssd_combined_args& a) {
                <= 2 * bh * ncw * a.headdim * a.dstate;
     };
     const bool p32 = a.headdim == 32;         // a whole head is what half of one of 64 is
+    // chunks per segment: whole chunks of the layer (see rising())
+    const int64_t sub = a.chunk_size / Q;
+    auto seg_chunks = [&](int64_t seg) { return seg == 1 ? nc : (nc + seg * sub - 1) / (seg * sub) * sub; };
     const int force = dispatch_override(M2_KNOB_LAYER);
     if (force == 3 || !fits(nc)) return none;
     if (force) {
-        const int64_t seg = force >= 4 ? force / 2 : 1, cps = (nc + seg - 1) / seg;
+        const int64_t cps = seg_chunks(force >= 4 ? force / 2 : 1);
         if (!fits(cps)) return none;
         return {p32 ? 1 : force >= 4 ? 1 + (force & 1) : force, cps, (nc + cps - 1) / cps};
     }
@@ -911,7 +1054,7 @@ static WalkPlan walk_plan(const m2_ssd_combined_args& a) {
     double tb = 0.0;
     for (int parts = 1; parts <= (p32 ? 1 : 2); ++parts)
         for (int64_t seg = 1; seg <= 32 && seg <= nc; ++seg) {
-            const int64_t cps = (nc + seg - 1) / seg;
+            const int64_t cps = seg_chunks(seg);
             // segments only where the chains leave CUs idle
             if (seg > 1 && (cps < 2 || !fits(cps) || bh * parts >= cu_count())) break;
             const double t = walk_cost(bh, nc, cps, parts, p32 || parts == 2, (int)a.dstate, a.z != nullptr, cu_count());
@@ -964,11 +1107,11 @@ int launch_ssd_walk(const m2_ssd_combined_args& a, const float* dA, const float*
     M2_REQUIRE(p.parts > 0, M2_ERR_UNSUPPORTED, "ssd_walk: unsupported shape / dtype");
     WalkArgs k{};
     k.x = (const bf16*)a.x; k.B = (const bf16*)a.B; k.C = (const bf16*)a.C; k.z = (const bf16*)a.z;
-    k.cb = (const bf16*)cb; k.dA = dA; k.dt = dt; k.wts = wts; k.D = a.D; k.init = a.initial_states;
+    k.cb = (const bf16*)cb; k.dA = dA; k.dt = dt; k.wts = wts; k.A = a.A; k.D = a.D; k.init = a.initial_states;
     k.out = a.out; k.fin = a.final_states;
     k.L = (int)a.seqlen; k.H = (int)a.nheads; k.G = (int)a.ngroups;
     k.P = (int)a.headdim; k.nc = (int)((a.seqlen + Q - 1) / Q); k.D_has_hdim = a.D_has_hdim;
-    k.cps = (int)p.cps; k.nseg = (int)p.nseg;
+    k.cps = (int)p.cps; k.nseg = (int)p.nseg; k.sub = (int)(a.chunk_size / Q);
     const int64_t bh = a.batch * a.nheads, nwork = bh * p.nseg * p.parts;
     M2_REQUIRE(nwork < (1ll << 31), M2_ERR_UNSUPPORTED, "ssd_walk: too many workgroups");
     // behind CB, 256-byte aligned: the segment states, then their decays

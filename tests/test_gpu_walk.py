@@ -7,6 +7,9 @@ per head dim, rising dA_cumsum; and the plan the library picks by itself.
 Tolerance: the bf16 bar of the layer, 2e-2 of the RMS (it holds CB and the
 states entering each chunk in bf16, as the other paths do)."""
 
+import contextlib
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -47,6 +50,19 @@ def _inputs(b, Lq, H, G, N, Q, init, z, dhp, P=64, *, seed):
     return d, t
 
 
+def _plan(t, chunk, plan=None):
+    """(segments, workgroups per head) of the walk that the library runs, (0, 0) where
+    it does not."""
+    b, Lq, H, P = t["x"].shape
+    args = L.SsdCombinedArgs(
+        batch=b, seqlen=Lq, nheads=H, headdim=P, ngroups=t["B"].shape[2], dstate=t["B"].shape[3],
+        chunk_size=chunk, dtype=L.dtype_code(t["x"], "x"), dt_dtype=L.dtype_code(t["dt"], "dt"),
+        dt_softplus=1, dt_min=0.0, dt_max=float("inf"), z=L.ptr(t.get("z")))
+    with L.dispatch_override("layer", plan) if plan else contextlib.nullcontext():
+        p = L.load_library().m2_ssd_combined_plan(ctypes.byref(args))
+    return (p // 2, p % 2 + 1) if p else (0, 0)
+
+
 def _check_all(t, d, plans, decay_clamp=False, **kw):
     want = O.ssd_combined(io_dtype="bf16", decay_clamp=decay_clamp, **d, **kw)
     for plan in plans:
@@ -67,17 +83,50 @@ def test_walk_matches_oracle(shape):
     _check_all(t, d, PLANS + [None], chunk_size=shape[5], dt_softplus=True, return_final_states=True)
 
 
-def test_walk_rising_dA():
-    """A > 0: dA_cumsum rises, and the chunk states' decay is clamped at 0 chunk by
-    chunk, so the oracle runs the walk's chunks of 64.  The oracle rounds C h_c to
-    bf16 before the factor exp(dA): with A <= 16 / 2000 and dt' < 2 a chunk's dA
-    stays below 64 * 2 * 8e-3 = 1, so that rounding grows to at most 2^-9 e = 5.4e-3
-    of the term (A 20 times larger, exp(dA) to e^20, put it at 4.9e-2)."""
-    d, t = _inputs(1, 300, 4, 2, 128, 64, False, False, False, seed=5)
-    d["A"] = np.abs(d["A"] / 2000).astype(np.float32)
+# A > 0: (L, dstate, chunk, head dim, init, z, plan, segments, workgroups per head)
+RISING = [
+    (300, 128, 64, 64, False, False, "walk", 1, 1),
+    (700, 128, 128, 64, False, False, "walk", 1, 1),
+    (700, 128, 128, 64, True, False, "walk_half", 1, 2),
+    (700, 128, 128, 64, True, False, "walk_x3", 3, 1),
+    (705, 64, 128, 64, False, True, "walk_half_x2", 2, 2),
+    (640, 64, 256, 64, True, False, "walk", 1, 1),
+    (1000, 256, 128, 64, True, False, "walk", 1, 1),
+    (1000, 256, 128, 64, False, False, "walk_half_x2", 2, 2),
+    (1000, 256, 128, 64, True, True, "walk_x2", 2, 1),
+    (1100, 128, 256, 32, False, False, "walk", 1, 1),
+    (1100, 128, 256, 32, True, False, "walk_x2", 2, 1),
+    (1100, 256, 256, 32, True, False, "walk", 1, 1),
+    (1100, 64, 128, 32, True, False, "walk_x2", 2, 1),
+]
+
+
+@pytest.mark.parametrize("case", RISING, ids=lambda c: "-".join(str(v) for v in c))
+def test_walk_rising_dA(case):
+    """A > 0 (all heads but one): dA_cumsum rises, and the chunk states' weights are
+    clamped chunk by chunk of the layer (64, 128 or 256 positions) while the outputs
+    are not, whatever the walk's own chunks are.  The other path computes the same: it
+    rounds C h to bf16 before exp(dA) and the intra-chunk CB of positions that the walk
+    carries in a bf16 state, 2^-9 = 2e-3 of a part of the result; its states hold
+    no rounding but that of w x, 2^-17 = 8e-6.  Weights clamped over 64 positions move
+    the states by 7e-2 (chunk 128, max over RMS) and more."""
+    Lq, N, Q, P, init, z, plan, nseg, parts = case
+    announce("rising", case)
+    d, t = _inputs(1, Lq, 4, 1, N, Q, init, z, False, P, seed=5)
+    d["A"] = np.abs(d["A"] / 500).astype(np.float32)
+    d["A"][1] *= -100
     t["A"] = dev(d["A"])
-    _check_all(t, d, ["walk", "walk_half_x3"], decay_clamp=True, chunk_size=64, dt_softplus=True,
-               return_final_states=True)
+    kw = dict(chunk_size=Q, dt_softplus=True, return_final_states=True)
+    assert _plan(t, Q, plan) == (nseg, parts)
+    _check_all(t, d, [plan], decay_clamp=True, **dict(kw, chunk_size=Q if P == 32 else min(Q, 128)))
+    outs = {}
+    for p in ("two_pass", plan):
+        with L.dispatch_override("layer", p):
+            outs[p] = mamba_chunk_scan_combined_fwd(**t, **kw)
+    for what, a, b, tol in zip(("out", "final"), outs["two_pass"], outs[plan], (2e-3, 8e-6)):
+        err = float((a.double() - b.double()).norm() / a.double().norm())
+        print(f"  {what} against the two passes: {err:.2e}", flush=True)
+        assert err <= tol
 
 
 def test_signed_dt_keeps_the_two_passes():
