@@ -164,7 +164,8 @@ int launch_rms_norm_gated(const m2_rms_norm_gated_args& a, hipStream_t s) {
         const int64_t n4 = a.group_size / 4;
         // Threads per (row, group), measured with a bf16 z or a residual, bf16 out
         // (us before -> now).  Groups of up to 1024: one chunk per thread at every
-        // row count (768: 4.2 -> 3.1 at 16 rows, 10.3 -> 9.2 at 4096).  Up to one
+        // row count (768: 4.2 -> 3.1 at 16 rows, 10.3 -> 9.2 at 4096; 4096 rows of 8
+        // groups of 512 32.1 -> 30.0, 44 with 256 threads, half of them idle).  Up to one
         // group per CU a workgroup's own latency is the time, so as many threads
         // as there are chunks (16 rows: 2560 4.9 -> 4.0, 5120 7.0 -> 4.8, 8192 9.6
         // -> 6.1).  More groups want fewer threads with two to four chunks in
@@ -173,6 +174,7 @@ int launch_rms_norm_gated(const m2_rms_norm_gated_args& a, hipStream_t s) {
         const bool few = nblocks <= cu_count();
 #define M2_NORM(NT, E) hipLaunchKernelGGL((k_rms_norm<NT, E, 4>), grid, dim3(NT), 0, s, k)
         if (n4 <= 64) M2_NORM(64, 1);
+        else if (n4 <= 128) M2_NORM(128, 1);
         else if (n4 <= 256) M2_NORM(256, 1);
         else if (few && n4 <= 1024) M2_NORM(1024, 1);
         else if (few && n4 <= 2048) M2_NORM(1024, 2);

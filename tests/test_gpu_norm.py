@@ -167,7 +167,7 @@ def test_norm_sweep(case):
 
 
 @pytest.mark.parametrize("rows", [2, 300])
-@pytest.mark.parametrize("d", [256, 260, 1024, 1028, 2048, 2052, 3072, 3076, 4096, 4100, 8192, 8196, 16384, 16396])
+@pytest.mark.parametrize("d", [256, 260, 512, 516, 1024, 1028, 2048, 2052, 3072, 3076, 4096, 4100, 8192, 8196, 16384, 16396])
 def test_threads_per_group(rows, d):
     """The sizes at which the launcher changes the threads of a group, with fewer
     and more rows than CUs: gate before the norm, and the residual add."""
