@@ -4,8 +4,8 @@
 // A decode step reads every projection weight once per token, so these
 // products are HBM-bound on the weights (M * K * N MACs for 2 * K * N bytes).
 // The weights are K-contiguous ([N, K], the layout torch.nn.functional.linear
-// takes).  Up to 16 rows run k_skinny_stream (below); k_skinny_gemm takes the
-// rest: each lane loads 8 consecutive k of one output column as one
+// takes).  Up to 16 rows run k_skinny_stream (below) unless K is short;
+// k_skinny_gemm takes the rest: each lane loads 8 consecutive k of one output column as one
 // 16-byte access, which is exactly a 16x16x32 bf16 MFMA's B-operand fragment.
 // One workgroup per 16 output columns (fewer where that leaves CUs idle); its
 // 4, 8 or 16 wavefronts (enough for ~2048 over the chip) split K and meet in
@@ -477,6 +477,23 @@ void launch_mt(const GemmArgs& k, int64_t ngroups, hipStream_t s) {
     }
 }
 
+// Where k_skinny_stream is the faster of the two at up to 16 rows, over 13 K from 64
+// to 8192, 10 N from 256 to 50288 and 1 to 16 rows (us k_skinny_gemm /
+// k_skinny_stream, weights past the cache).  By N and K alone, so that a row's result
+// does not depend on how many rows come with it.
+bool stream_faster(const GemmArgs& k, int64_t cus) {
+    // two or three column tiles per workgroup, one round of them: from 384 on (4
+    // rows: 384 x 6448 4.0 / 3.8, 512 x 10576 5.1 / 4.4; 64 x 6448 2.9 / 3.1)
+    if (k.N > 16 * cus && k.N <= 48 * cus) return k.K >= 384;
+    // one tile, or several rounds: short K ranges pay neither for 16 wavefronts (4
+    // rows: 512 x 2048 3.3 / 3.5, 768 x 3352 3.9 / 3.8) nor for every round's start
+    // (64 x 50288 5.4 / 11.3, 512 x 50288 12.8 / 17.0).  From 768 on it depends on
+    // the rows, as k_skinny_gemm reads x again for every 16 columns: 768 x 50288 19.3 /
+    // 21.9 at 4, 25.9 / 22.4 at 16; so does K 2048, whose rows 4 KB apart meet on the
+    // same memory channels: 2048 x 8192 9.4 / 10.0 and 12.0 / 10.3
+    return k.K >= 768;
+}
+
 // k_skinny_stream for up to 16 rows and K up to 8192 (8 units of x fragments in
 // each of 16 wavefronts): false where it does not apply.  8 wavefronts with
 // twice the ring each where several column tiles follow each other and a K range
@@ -498,6 +515,7 @@ bool launch_stream_pu(const GemmArgs& k, int pu, const dim3& grid, hipStream_t s
 bool launch_stream(GemmArgs k, hipStream_t s) {
     const int64_t cus = m2::cu_count();
     if (k.M > 16 || k.K > 8192 || k.ldx >= (1 << 24) || k.ldw >= (1 << 24)) return false;   // 32-bit offsets
+    if (!stream_faster(k, cus)) return false;
     // columns per workgroup: as even over whole rounds of the CUs as up to three
     // tiles allow, at least 4
     const int64_t r = (k.N + 48 * cus - 1) / (48 * cus);

@@ -59,7 +59,11 @@ def test_strided_x_and_errors():
 # strides.  |error| <= K 2^-24 sum |x w| bounds any order of a float32 sum of K
 # products.
 STREAM = [(1, 8, 1), (16, 64, 4), (3, 72, 700), (15, 1000, 4097), (16, 768, 12301), (2, 2568, 513),
-          (7, 3080, 8209), (9, 6144, 300), (16, 8192, 5000), (13, 8200, 77), (5, 1536, 24600)]
+          (7, 3080, 8209), (9, 6144, 300), (16, 8192, 5000), (13, 8200, 77), (5, 1536, 24600),
+          # and on either side of each line of the rule that picks it: K 384 between 16
+          # and 48 columns per CU (256 of them), K 768 elsewhere
+          (5, 376, 4097), (16, 392, 4099), (2, 760, 700), (1, 776, 3), (10, 384, 12288), (11, 760, 12289),
+          (7, 776, 12289), (3, 768, 4096)]
 
 
 @pytest.mark.parametrize("M,K,N", STREAM)
