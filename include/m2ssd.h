@@ -224,7 +224,7 @@ typedef struct {
 size_t m2_ssd_combined_workspace_size(const m2_ssd_combined_args* a);
 
 /* The kernels m2_ssd_combined runs for these sizes, types and flags (pointers are
- * only tested for NULL): 0 the staged or two-pass path; else the one-pass walk,
+ * only tested for NULL, x and B for 16-byte alignment): 0 the staged or two-pass path; else the one-pass walk,
  * 2 s + p - 1 for s segments of a chain and p workgroups per head.  For
  * measurements. */
 int m2_ssd_combined_plan(const m2_ssd_combined_args* a);

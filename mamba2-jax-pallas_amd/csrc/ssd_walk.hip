@@ -1027,6 +1027,8 @@ static WalkPlan walk_plan(const m2_ssd_combined_args& a) {
     if (a.dstate != 64 && a.dstate != 128 && a.dstate != 256) return none;
     if (a.ngroups <= 0 || a.nheads % a.ngroups || a.chunk_size % Q) return none;
     if (a.headdim == 64 && a.chunk_size > 2 * Q) return none;       // state_path's rising chains
+    // x and B come by 16-byte direct loads
+    if (((uintptr_t)a.x | (uintptr_t)a.B) & 15) return none;
     if (dispatch_override(M2_KNOB_STATES_SPLIT)) return none;
     // dt' >= 0, so that dA is monotonic: the intra-chunk weights' two factors need
     // it, and it leaves the clamp of the state weights to the sign of A (rising())

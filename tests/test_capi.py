@@ -165,3 +165,19 @@ def test_dispatch_override_hook_without_gpu():
     hdr = open(HEADER).read()
     defs = {n.lower(): int(v) for n, v in re.findall(r"#define M2_KNOB_(\w+)\s+(\d+)", hdr)}
     assert defs == {k: v[0] for k, v in L.KNOBS.items()}
+
+
+@pytest.mark.parametrize("headdim", [32, 64])
+def test_walk_needs_aligned_rows(headdim):
+    """The one-pass walk brings x and B into LDS by 16-byte direct loads: a call whose
+    pointers are not aligned to that keeps the kernels it always had (at head dim 32
+    ordinary vector loads, which take any alignment)."""
+    def plan(**ptrs):
+        a = L.SsdCombinedArgs(batch=1, seqlen=4096, nheads=128, headdim=headdim, ngroups=8, dstate=128,
+                              chunk_size=128, dtype=1, dt_dtype=1, dt_softplus=1, dt_min=0.0,
+                              dt_max=float("inf"), **ptrs)
+        return L.load_library().m2_ssd_combined_plan(ctypes.byref(a))
+    assert plan(x=4096, B=8192) > 0
+    for off in (2, 4, 8):
+        assert plan(x=4096 + off, B=8192) == 0
+        assert plan(x=4096, B=8192 + off) == 0
