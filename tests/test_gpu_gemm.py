@@ -79,9 +79,29 @@ def test_skinny_stream(M, K, N):
     err = (y.double() - ref).abs()
     print(f"  max err / bound {float((err / bound).max()):.3f}", flush=True)
     assert bool((err <= bound).all())
-    # rows past M and the columns of other workgroups are never written
+    # a row's result does not depend on the rows beside it
     z = linear_skinny(x[:1], w, b, out_dtype=torch.float32)
     assert torch.equal(z[0], y[0])
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,K,N", STREAM)
+def test_skinny_stream_writes_only_its_rows(M, K, N, dt):
+    """y as rows of a larger buffer: nothing outside the M x N results changes, and
+    each column's is stored (a workgroup's store into a neighbour's would show in
+    the comparison with the contiguous call)."""
+    announce("skinny stream stores", M, K, N, dt)
+    g = torch.Generator(device="cuda").manual_seed(M + K + N)
+    x = torch.randn((M, K), generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randn((N, K), generator=g, device="cuda").to(torch.bfloat16)
+    buf = torch.full((M + 18, N + 40), -12345.0, device="cuda", dtype=dt)
+    y = buf[1:M + 1, 8:8 + N]
+    a = L.SkinnyGemmArgs(x=L.ptr(x), w=L.ptr(w), y=y.data_ptr(), M=M, N=N, K=K, ldx=K, ldw=K,
+                         ldy=N + 40, x_dtype=L.M2_BF16, w_dtype=L.M2_BF16, y_dtype=L.dtype_code(buf, "y"))
+    L.call("m2_skinny_gemm", a, L.stream_of(buf.device))
+    assert torch.equal(y, linear_skinny(x, w, None, out_dtype=dt))
+    y.fill_(-12345.0)
+    assert bool((buf == -12345.0).all())
 
 
 # ---------------------------------------------------------------------------

@@ -1,8 +1,9 @@
 """The one-pass layer (csrc/ssd_walk.hip) against the oracle where it can go
 wrong: one position to a few chunks of 64 with every remainder, each dstate, a
-whole head or half of one per workgroup, chains cut into segments (fewer chunks
-than asked for, a last segment that is shorter), initial states, the z gate, D
-per head dim, rising dA_cumsum; and the plan the library picks by itself.
+whole head or half of one per workgroup, chains cut into segments (up to 32, a
+last one that is shorter; each forced plan is asked for by what it runs), initial
+states, the z gate, D per head dim, rising dA_cumsum; and the plan the library
+picks by itself.
 
 Tolerance: the bf16 bar of the layer, 2e-2 of the RMS (it holds CB and the
 states entering each chunk in bf16, as the other paths do)."""
@@ -22,20 +23,28 @@ from oracle import ssd_oracle as O
 
 pytestmark = pytest.mark.gpu
 
-PLANS = ["walk", "walk_half", "walk_x2", "walk_half_x3", "walk_x32"]
-# (batch, L, H, G, dstate, chunk, init, z, D per head dim[, head dim])
+# (batch, L, H, G, dstate, chunk, init, z, D per head dim[, head dim]) and, beside a
+# whole and half a head per workgroup, the cuts of its chains that the workspace holds:
+# {forced plan: (segments, workgroups per head) that it runs}
 SHAPES = [
-    (1, 1, 2, 1, 128, 128, False, False, False),
-    (2, 63, 4, 2, 64, 64, True, False, True),
-    (1, 64, 4, 1, 256, 128, True, True, False),
-    (1, 65, 2, 1, 128, 256, False, True, True),
-    (3, 130, 6, 2, 128, 128, True, False, False),
-    (1, 447, 4, 1, 256, 64, False, False, True),
-    (1, 1000, 5, 1, 64, 128, True, True, True),
-    (2, 1088, 4, 4, 128, 256, True, False, False),
-    (1, 65, 4, 2, 128, 256, True, True, False, 32),
-    (2, 700, 6, 1, 64, 128, False, False, True, 32),
-    (1, 1000, 4, 1, 256, 64, True, False, False, 32),
+    ((1, 1, 2, 1, 128, 128, False, False, False), {}),
+    ((2, 63, 4, 2, 64, 64, True, False, True), {}),
+    ((1, 64, 4, 1, 256, 128, True, True, False), {}),
+    ((1, 65, 2, 1, 128, 256, False, True, True), {}),
+    ((3, 130, 6, 2, 128, 128, True, False, False), {}),
+    ((1, 447, 4, 1, 256, 64, False, False, True),
+     {"walk_x2": (2, 1), "walk_half_x3": (3, 2), "walk_x5": (4, 1)}),
+    ((1, 1000, 5, 1, 64, 128, True, True, True), {"walk_x2": (2, 1), "walk_half_x3": (3, 2)}),
+    ((2, 1088, 4, 4, 128, 256, True, False, False), {"walk_x2": (2, 1)}),
+    ((1, 65, 4, 2, 128, 256, True, True, False, 32), {}),
+    ((2, 700, 6, 1, 64, 128, False, False, True, 32), {"walk_x2": (2, 1)}),
+    ((1, 1000, 4, 1, 256, 64, True, False, False, 32), {"walk_x2": (2, 1), "walk_x5": (4, 1)}),
+    ((1, 1000, 8, 1, 128, 128, True, False, True),
+     {"walk_x2": (2, 1), "walk_half_x3": (3, 2), "walk_x5": (4, 1)}),
+    ((2, 901, 4, 1, 128, 64, True, True, False), {"walk_x5": (5, 1), "walk_half_x5": (5, 2)}),
+    ((1, 2100, 6, 1, 128, 64, True, False, False, 32), {"walk_x3": (3, 1), "walk_x16": (11, 1)}),
+    # as many segments as there are, the last one shorter
+    ((1, 4090, 12, 1, 128, 64, True, False, False), {"walk_x32": (32, 1), "walk_half_x32": (32, 2)}),
 ]
 
 
@@ -66,7 +75,7 @@ def _plan(t, chunk, plan=None):
 def _check_all(t, d, plans, decay_clamp=False, **kw):
     want = O.ssd_combined(io_dtype="bf16", decay_clamp=decay_clamp, **d, **kw)
     for plan in plans:
-        announce("walk", plan)
+        announce("walk", plan, _plan(t, kw["chunk_size"], plan))
         if plan is None:
             got = mamba_chunk_scan_combined_fwd(**t, **kw)
         else:
@@ -76,11 +85,52 @@ def _check_all(t, d, plans, decay_clamp=False, **kw):
         check(got[1], want[1], TOL["bf16"], "final_states")
 
 
-@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "-".join(str(int(v)) for v in s))
-def test_walk_matches_oracle(shape):
+@pytest.mark.parametrize("shape,cuts", SHAPES, ids=lambda s: "-".join(str(int(v)) for v in s)
+                         if isinstance(s, tuple) else f"{len(s)}cuts")
+def test_walk_matches_oracle(shape, cuts):
     announce("walk shape", shape)
     d, t = _inputs(*shape, seed=sum(shape[:5]))
-    _check_all(t, d, PLANS + [None], chunk_size=shape[5], dt_softplus=True, return_final_states=True)
+    plans = {"walk": (1, 1), "walk_half": (1, 1 if t["x"].shape[3] == 32 else 2), **cuts}
+    for plan, runs in plans.items():
+        assert _plan(t, shape[5], plan) == runs, plan
+    _check_all(t, d, [*plans, None], chunk_size=shape[5], dt_softplus=True, return_final_states=True)
+
+
+# (shape, plan): long chains, every dstate and head dim, cut or not
+LONG = [((1, 8192, 4, 2, 128, 128, True, False, False), "walk_half_x31"),
+        ((1, 8192, 4, 2, 128, 128, True, True, False), "walk_x16"),
+        ((1, 8192, 4, 2, 128, 128, True, False, False), "walk"),
+        ((1, 5000, 3, 1, 256, 128, True, False, False), "walk_x16"),
+        ((1, 5000, 3, 1, 256, 128, True, False, False), "walk_half_x3"),
+        ((1, 4100, 2, 1, 64, 64, True, False, True), "walk_x32"),
+        ((1, 4100, 6, 1, 128, 64, True, False, False, 32), "walk_x16"),
+        ((1, 4100, 6, 1, 256, 256, True, False, False, 32), "walk_x2")]
+
+
+@pytest.mark.parametrize("shape,plan", LONG, ids=lambda v: v if isinstance(v, str) else "-".join(str(int(i)) for i in v))
+def test_walk_against_the_other_path(shape, plan):
+    """Every row of y and every state row beside the other path's.  Both paths round
+    at 2^-9: CB, the state that enters a chunk, and (the other path) C h, none of them
+    to the same partial sums, so a row of y may differ by two such roundings, 2^-8, of
+    itself or, where its terms cancel, of a typical row; over all rows, whose roundings
+    are independent and most of whose value is D x, 1e-4 (2e-5 seen).  The states see
+    the rounding of w x alone, 2^-17, in different chunks."""
+    announce("walk against", shape, plan)
+    d, t = _inputs(*shape, seed=3)
+    kw = dict(chunk_size=shape[5], dt_softplus=True, return_final_states=True)
+    nseg, parts = _plan(t, shape[5], plan)
+    assert nseg > 1 or plan == "walk"
+    outs = {}
+    for p in ("two_pass", plan):
+        with L.dispatch_override("layer", p):
+            outs[p] = [v.double() for v in mamba_chunk_scan_combined_fwd(**t, **kw)]
+    for what, a, b, tol, all_ in zip(("out", "final"), outs["two_pass"], outs[plan],
+                                     (2.0 ** -8, 2.0 ** -16), (1e-4, 2.0 ** -17)):
+        an, rms = a.norm(dim=-1), a.norm() / a[..., 0].numel() ** 0.5
+        err = (a - b).norm(dim=-1) / (an + rms)
+        total = float((a - b).norm() / a.norm())
+        print(f"  {what}: worst row {float(err.max()):.2e}, all {total:.2e}", flush=True)
+        assert float(err.max()) <= tol and total <= all_
 
 
 # A > 0: (L, dstate, chunk, head dim, init, z, plan, segments, workgroups per head)
@@ -145,9 +195,10 @@ def test_signed_dt_keeps_the_two_passes():
 
 def test_walk_large_decay():
     """|dA| past 500 within a chunk: the decay factors underflow, none overflows."""
-    d, t = _inputs(1, 300, 4, 1, 128, 128, True, False, False, seed=6)
+    d, t = _inputs(1, 700, 4, 1, 128, 128, True, False, False, seed=6)
     d["A"] = (d["A"] * 40).astype(np.float32)
     t["A"] = dev(d["A"])
+    assert _plan(t, 128, "walk_half_x3") == (3, 2)
     _check_all(t, d, ["walk", "walk_half_x3"], chunk_size=128, dt_softplus=True,
                return_final_states=True)
 
