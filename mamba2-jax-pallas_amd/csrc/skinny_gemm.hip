@@ -498,18 +498,16 @@ bool stream_faster(const GemmArgs& k, int64_t cus) {
 // each of 16 wavefronts): false where it does not apply.  8 wavefronts with
 // twice the ring each where several column tiles follow each other and a K range
 // is at most 6 units; 16 for a single tile, whose loads all go out at once.
-template <int CT, int NW, int D>
+// Units of a K range by the wavefronts: 1 to 6 with 8; with 16 4 to 8 (K behind 8
+// wavefronts' 48 units), or 1 to 8 for a single tile.
+template <int CT, int NW, int D, int PU = (NW == 16 && CT > 1) ? 4 : 1>
 bool launch_stream_pu(const GemmArgs& k, int pu, const dim3& grid, hipStream_t s) {
-#define M2_STREAM_PU(V)                                                                    \
-    case V:                                                                                \
-        hipLaunchKernelGGL((k_skinny_stream<CT, V, NW, D>), grid, dim3(NW * 64), 0, s, k); \
+    if constexpr (PU <= (NW == 16 ? 8 : 6)) {
+        if (pu != PU) return launch_stream_pu<CT, NW, D, PU + 1>(k, pu, grid, s);
+        hipLaunchKernelGGL((k_skinny_stream<CT, PU, NW, D>), grid, dim3(NW * 64), 0, s, k);
         return true;
-    switch (pu) {
-        M2_STREAM_PU(1) M2_STREAM_PU(2) M2_STREAM_PU(3) M2_STREAM_PU(4) M2_STREAM_PU(5) M2_STREAM_PU(6)
-        M2_STREAM_PU(7) M2_STREAM_PU(8)
-        default: return false;
     }
-#undef M2_STREAM_PU
+    return false;
 }
 
 bool launch_stream(GemmArgs k, hipStream_t s) {
