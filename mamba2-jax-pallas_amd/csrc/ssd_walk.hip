@@ -34,7 +34,7 @@
 // CB that each workgroup reads from L2 are 37 of its 42 KB.  The layer at 128
 // heads, dstate 128, 4096 tokens takes 79 us (2.7 TB/s over its compulsory 223
 // MB) against 107 for the state pass and the scan, at 256 heads, dstate 256, 182
-// against 276, at 24 heads and 30011 tokens 143 against 364 in 10 segments.
+// against 276, at 24 heads and 30011 tokens 135 against 364 in 10 segments.
 // Chunks of 128 would halve the barriers, but their operands do not fit LDS
 // twice at dstate 256.  One wavefront for carry and intra together: 93 against
 // 82 us at the first shape; loads issued by two wavefronts: 100.
@@ -798,6 +798,9 @@ M2_DEV void state_path(const WalkArgs& a, const char* ring, char* hs, int sw, in
     if (a.fin && seg == a.nseg - 1) st.store(a.fin + st.off(bh, a.P, p0));
 }
 
+// (16 wavefronts leave a lane 128 registers: at dstate 256 with whole heads the
+// state wavefronts spill 14, 56 bytes of scratch, no other instance any.  The data
+// wavefronts must not: a scratch access would count in their waits.)
 template <int NS, int PT, bool HASZ, bool NTO>
 __global__ void __launch_bounds__(THREADS) k_ssd_walk(WalkArgs a) {
     typedef WCfg<NS, PT> S;
@@ -1012,7 +1015,7 @@ static double walk_cost(int64_t bh, int64_t nc, int64_t cps, int parts, bool hal
 // shapes (2 to 5120 chains, 38 to 30011 tokens, each dstate, some with z) the
 // choice loses 1 % on average against the best of every plan and path; the
 // widest gaps it decides: 2 heads x 20000 tokens 43 us against 162 for the two
-// passes, 24 x 30011 152 against 364, 256 x 8192 at dstate 256 394 against 485,
+// passes, 24 x 30011 135 against 364, 256 x 8192 at dstate 256 394 against 485,
 // and 320 x 4096 at dstate 128 257 against 239.
 static double two_pass_cost(const m2_ssd_combined_args& a) {
     const double x = 2.0 * a.batch * a.seqlen * a.nheads * 64, bc = 4.0 * a.batch * a.seqlen * a.ngroups * a.dstate;
